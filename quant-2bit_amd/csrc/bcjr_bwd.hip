@@ -1,4 +1,4 @@
-// Backward of the BCJR node: d seq for L = sum(g_soft * soft) + sum(g_logZ * logZ).
+// Backward of the BCJR node for kV <= 2 (bcjr_soft16.h runs kV = 4): d seq for L = sum(g_soft * soft) + sum(g_logZ * logZ).
 //
 // Replaces the analytic backward of BcjrForwardBackwardMonolithic
 // (src/bcjr/bcjr_monolithic.py:192-243), i.e. the eager autograd of
@@ -38,10 +38,6 @@
 
 namespace bcjr {
 
-// Unroll of the loop over a butterfly's outputs: full for 2 or 4 states.
-template <int R>
-constexpr int kOuterUnroll = R <= 4 ? R : 1;
-
 // A butterfly's slot entry: R (m~, mu) pairs, 8-byte aligned.  Each pair is
 // stored from the two registers the LDS read filled, so no register moves
 // assemble a wider store.
@@ -65,25 +61,14 @@ __device__ __forceinline__ void load_pairs(const float* src, float (&m)[R], floa
 }
 
 template <int KV, int V, int CODE, int UPT, int CU, int CUA>
-__global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_COL ? 3 : 1) void bcjr_bwd_kernel(BwdParams P) {
+__global__ __launch_bounds__(512, 1) void bcjr_bwd_kernel(BwdParams P) {
   constexpr int R = 1 << KV;
   // Butterflies whose slot inputs are in flight ahead of the beta sweep's use
   // (3 or 4 measured no faster at L=16: the HBM latency is already covered).
   constexpr int kSlotAhead = 2;
   using CT = CodeTraits<CODE>;
-  // Butterflies of 2 or 4 states run fully unrolled with their slot-side
-  // inputs prefetched in registers; 16-state butterflies loop over outputs and
-  // read those inputs from the slot as they go (the loop unrolled on the HYB
-  // column walk, whose LUT offsets are then immediates).
-  constexpr bool kPair = R <= 4;
-  static_assert((CU == 0 && CUA == 0) || kPair, "codeword cache is for butterflies of at most 4 states");
+  static_assert(R <= 4, "butterflies run fully unrolled, their slot inputs prefetched in registers");
   static_assert(CU <= UPT && CUA <= UPT, "at most UPT cached butterflies");
-  constexpr bool kCol = CODE == CODE_HYB_COL;  // HYB column walk: one butterfly per thread
-  static_assert(!kCol || (KV == 4 && UPT == 1), "the column walk is for L = 16, kV = 4");
-  constexpr bool kColUnroll = kCol;  // outputs unrolled: immediate LUT offsets
-  // Its alpha + mu sweep reads each state's emission and path feature from a
-  // per-step table (below).
-  constexpr bool kETab = kColUnroll;
 
   extern __shared__ __align__(16) unsigned char smem[];
   const int L = P.L, N = P.N;
@@ -93,18 +78,12 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
   const uint32_t ANT = opaque_uniform(CT::A * (uint32_t)NT);  // hash offset of p * NT
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int lane = tid & 63, wave = tid >> 6, nwaves = nthr >> 6;
-  // The column-walk instance gives thread tid butterfly col_walk_unit(tid), so
-  // that a half-wave's LUT reads hit distinct banks (the host picks the state
-  // swizzle for that lane map); elsewhere u = tid.
-  const int utid = kColUnroll ? (int)col_walk_unit((uint32_t)tid) : tid;
   const Swizzle swz = P.swz;
 
-  // LDS: the (m~, mu) pairs sit at byte kPairBase (0, or 16 KiB behind the
-  // column walk's tables), so a pair's byte address is kPairBase plus 8 times
-  // its element index.
-  constexpr uint32_t kPairBase = kETab ? 16384u : 0u;
-  float2* mm = reinterpret_cast<float2*>(smem + kPairBase);                    // NT (m~, mu) then (n~, nu)
-  double* cvec = reinterpret_cast<double*>(smem + kPairBase + (size_t)8 * NT);  // N  C_{t-1}
+  // LDS: the (m~, mu) pairs come first, so a pair's byte address is 8 times its
+  // element index.
+  float2* mm = reinterpret_cast<float2*>(smem);                     // NT (m~, mu) then (n~, nu)
+  double* cvec = reinterpret_cast<double*>(smem + (size_t)8 * NT);  // N  C_{t-1}
   float* wmax = reinterpret_cast<float*>(cvec + ((N + 1) & ~1));    // 2*kMaxWaves
   float* wsum = wmax + 2 * kMaxWaves;                               // 2*kMaxWaves
   // Last wsum word: the block-wide input flag (at most 8 waves use wsum, launch
@@ -113,58 +92,14 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
   float* wbuf = wsum + 2 * kMaxWaves;                               // N*V
   float* gbuf = wbuf + N * V;                                       // N*V
   float* apart = gbuf + N * V;                                      // 2*nwaves*(V+1) per-wave partials
-  // HYB: signed LUT (code_hyb_signed), 8-byte aligned; kETab: the column walk's
-  // per-step tables at byte 0.
-  float* lut = kETab ? reinterpret_cast<float*>(smem)
-                     : reinterpret_cast<float*>(smem) +
-                           ((apart + 2 * nwaves * (V + 1) - reinterpret_cast<float*>(smem) + 1) & ~1);
+  // HYB: signed LUT (code_hyb_signed), 8-byte aligned
+  float* lut = reinterpret_cast<float*>(smem) +
+               ((apart + 2 * nwaves * (V + 1) - reinterpret_cast<float*>(smem) + 1) & ~1);
 
   if constexpr (CODE == CODE_HYB) {
     stage_hyb_signed(reinterpret_cast<float2*>(lut), P.table, P.Q, tid, nthr);
     __syncthreads();
   }
-  const unsigned char* lutb = reinterpret_cast<const unsigned char*>(lut);
-  // Table of the column-walk alpha + mu sweep, in the LUT's place until the beta
-  // sweep stages the LUT: per step, the float2 at entry k of the column-walk
-  // layout (32 rows of 64, rows 16..31 repeating 0..15) is (-|d|^2, sg . h) of
-  // that LUT entry h, d = h ssk + nw_t, so a state's pair sits at the byte its
-  // codeword has in the LUT.  The kernel runs 256 threads here; thread tid forms
-  // entries tid + 256j (j < 4) and their row copies, reading the codewords from
-  // the (2^Q, 2) table as stage_hyb_col does.
-  auto load_codewords = [&](float (&h)[4][2]) {
-    const int ncol = 1 << (P.Q - 3), mask = (1 << P.Q) - 1;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = tid + 256 * j, col = k & 63, i = col + ncol * (k >> 6), ie = i & mask;
-      h[j][0] = col < ncol ? P.table[2 * ie] : 0.0f;
-      const float y = col < ncol ? P.table[2 * ie + 1] : 0.0f;
-      h[j][1] = (i >> P.Q) ? -y : y;
-    }
-  };
-  auto build_etab = [&](const float (&h)[4][2], const float (&nw)[V], const float (&sg)[V], float ssk) {
-    float2* et = reinterpret_cast<float2*>(lut);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float e = 0.0f, f = 0.0f;
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const float d = fmaf(h[j][v], ssk, nw[v]);
-        e = fmaf(-d, d, e);
-        f = fmaf(sg[v], h[j][v], f);
-      }
-      const int k = tid + 256 * j;
-      et[k] = make_float2(e, f);
-      et[k + 1024] = make_float2(e, f);
-    }
-  };
-  // Column-walk bases of this thread's butterfly u = utid, input c (state R*u + c),
-  // for the beta sweep; the alpha sweep forms its output's base as it goes.
-  uint32_t cbs[kCol ? R : 1];
-  if constexpr (kCol) {
-#pragma unroll
-    for (int c = 0; c < R; ++c) cbs[c] = hyb_col_base((uint32_t)(R * min(utid, NB - 1) + c), P.Q);
-  }
-
   // Raw codewords h of this thread's first NC butterflies (hcx[i][p][c] for
   // state p*NT + R*u + c); the others are hashed per state.  Each sweep fills
   // its own cache when it starts (CUA butterflies for alpha + mu, CU for beta
@@ -175,7 +110,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
     constexpr int NC = decltype(count_tag)::value;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-      const int u = min(opaque(utid) + i * nthr, NB - 1);
+      const int u = min(opaque(tid) + i * nthr, NB - 1);
       const uint32_t xu = CT::A * (uint32_t)(R * u) + CT::B;
 #pragma unroll
       for (int p = 0; p < R; ++p)
@@ -186,12 +121,12 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
     }
   };
 
-  // Byte address of slot k of butterfly utid + i*nthr at rotation rho:
-  // 8 S(rotr(utid + i*nthr + k*NB)) = yb ^ unit_off(i) ^ slot_off(k), the last
-  // two uniform (utid, i*nthr and k*NB occupy disjoint bits; S and rotr are
+  // Byte address of slot k of butterfly tid + i*nthr at rotation rho:
+  // 8 S(rotr(tid + i*nthr + k*NB)) = yb ^ unit_off(i) ^ slot_off(k), the last
+  // two uniform (tid, i*nthr and k*NB occupy disjoint bits; S and rotr are
   // linear).
   auto base_off = [&](int rho) -> uint32_t {
-    return swizzle(rotr_bits((uint32_t)min(utid, NB - 1), rho, nb), swz) << 3;
+    return swizzle(rotr_bits((uint32_t)min(tid, NB - 1), rho, nb), swz) << 3;
   };
   auto unit_off = [&](int i, int rho) -> uint32_t {
     return swizzle(rotr_bits((uint32_t)(i * nthr), rho, nb), swz) << 3;
@@ -199,7 +134,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
   auto slot_off = [&](int k, int rho) -> uint32_t {
     return swizzle(rotr_bits((uint32_t)(k * NB), rho, nb), swz) << 3;
   };
-  auto lds_pair = [&](uint32_t off) -> float2& { return *reinterpret_cast<float2*>(smem + kPairBase + off); };
+  auto lds_pair = [&](uint32_t off) -> float2& { return *reinterpret_cast<float2*>(smem + off); };
 
   if (tid == 0) *bflag = 0;
   __syncthreads();
@@ -256,9 +191,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
       // --------------------------- alpha + mu sweep ----------------------------
       float hca[CUA > 0 ? CUA : 1][CUA > 0 ? R : 1][CUA > 0 ? R : 1][V];
       fill_cache(hca, std::integral_constant<int, CUA>{});
-      // kETab: this thread's 4 LUT entries for the per-step tables, held over the sweep
-      float hE[4][2];
-      if constexpr (kETab) load_codewords(hE);
       double C = 0.0;  // C_{t-1}
       int k = 0;
       int rho = nb - KV;  // kV * (t - 1) mod nb at t = 0
@@ -276,41 +208,21 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
           nw[v] = -wbuf[t * V + v] * sk;
           sg[v] = CT::kSigma * gbuf[t * V + v];  // f = g . c = sg . h
         }
-        if constexpr (kETab) {  // every wave has left step t-1's table (barrier at its end)
-          build_etab(hE, nw, sg, ssk);
-          __syncthreads();
-        }
         const uint32_t yb = base_off(rho);
         uint32_t Ku[UPT], Kk[R];  // uniform per step
 #pragma unroll
         for (int i = 0; i < UPT; ++i) Ku[i] = unit_off(i, rho);
-        if constexpr (kPair) {
 #pragma unroll
-          for (int c = 0; c < R; ++c) Kk[c] = slot_off(c, rho);
-        }
-        auto koff = [&](int c) -> uint32_t {
-          if constexpr (kPair) {
-            return Kk[c];
-          } else {
-            return slot_off(c, rho);
-          }
-        };
+        for (int c = 0; c < R; ++c) Kk[c] = slot_off(c, rho);
 
         // Output r of butterfly u: m~ and mu of state R*u + r from the shifted
         // inputs m[p] (maximum 0) and the raw mu inputs; returns the group sum.
-        // cb: the column-walk base of state R*u + r (kCol only).
         auto alpha_out = [&](auto shift_tag, int i, int r, uint32_t xu, int u, const float (&m)[R],
-                             const float (&mui)[R], float oout, float& mo, float& muo, uint32_t cb) -> float {
+                             const float (&mui)[R], float oout, float& mo, float& muo) -> float {
           constexpr bool SHIFT = decltype(shift_tag)::value;
           float a[R], phi[R];
 #pragma unroll
           for (int p = 0; p < R; ++p) {
-            if constexpr (kETab) {
-              const float2 ef = hyb_col_read(lutb, cb + hyb_col_step(p, r));
-              a[p] = m[p] + ef.x;
-              phi[p] = mui[p] + ef.y;
-              continue;
-            }
             float h[V];
             if (i < CUA) {
 #pragma unroll
@@ -351,7 +263,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
           const uint32_t yi = yb ^ Ku[i];
 #pragma unroll
           for (int p = 0; p < R; ++p) {
-            const float2 v2 = lds_pair(yi ^ koff(p));
+            const float2 v2 = lds_pair(yi ^ Kk[p]);
             m[p] = v2.x;
             mu[p] = v2.y;
           }
@@ -363,7 +275,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         float tmax = -INFINITY;
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
-          const int q = utid + i * nthr;
+          const int q = tid + i * nthr;
           float mi[R], mui[R];
 #pragma unroll
           for (int p = 0; p < R; ++p) {
@@ -384,59 +296,25 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
             const uint32_t xu = CT::A * (uint32_t)(R * u) + CT::B;
             const float oout = sh + O;
             const uint32_t yi = yb ^ Ku[i];
-            if constexpr (kPair) {
+            {
               float mo[R], muo[R], smin = 0.0f;
 #pragma unroll
               for (int r = 0; r < R; ++r) {
-                const float s = alpha_out(Fast{}, i, r, xu, u, m, mui, oout, mo[r], muo[r], 0u);
+                const float s = alpha_out(Fast{}, i, r, xu, u, m, mui, oout, mo[r], muo[r]);
                 smin = r ? fminf(smin, s) : s;
               }
               if constexpr (!EXACT) {
                 if (smin < kUnderflow) {
 #pragma unroll
                   for (int r = 0; r < R; ++r)
-                    alpha_out(std::true_type{}, i, r, xu, u, m, mui, oout, mo[r], muo[r], 0u);
+                    alpha_out(std::true_type{}, i, r, xu, u, m, mui, oout, mo[r], muo[r]);
                 }
               }
 #pragma unroll
               for (int r = 0; r < R; ++r) {
-                lds_pair(yi ^ koff(r)) = make_float2(mo[r], muo[r]);
+                lds_pair(yi ^ Kk[r]) = make_float2(mo[r], muo[r]);
               }
               tmax = max_with(tmax, mo);
-            } else if constexpr (kColUnroll) {
-              // Outputs unrolled, so every state's LUT offset is an immediate; a
-              // butterfly with an underflowed group is redone output by output
-              // (its inputs are in registers, its outputs overwrite the pairs).
-              float smin = 0.0f;
-#pragma unroll
-              for (int r = 0; r < R; ++r) {
-                float mo, muo;
-                const float s = alpha_out(Fast{}, i, r, xu, u, m, mui, oout, mo, muo, cbs[r]);
-                smin = r ? fminf(smin, s) : s;
-                lds_pair(yi ^ koff(r)) = make_float2(mo, muo);
-                tmax = vmax_raw(tmax, mo);
-              }
-              if constexpr (!EXACT) {
-                if (smin < kUnderflow) {
-#pragma unroll 1
-                  for (int r = 0; r < R; ++r) {
-                    float mo, muo;
-                    alpha_out(std::true_type{}, i, r, xu, u, m, mui, oout, mo, muo,
-                              hyb_col_base((uint32_t)(R * u + r), P.Q));
-                    lds_pair(yi ^ koff(r)) = make_float2(mo, muo);
-                    tmax = vmax_raw(tmax, mo);
-                  }
-                }
-              }
-            } else {
-#pragma unroll kOuterUnroll<R>
-              for (int r = 0; r < R; ++r) {
-                float mo, muo;
-                const float s = alpha_out(Fast{}, i, r, xu, u, m, mui, oout, mo, muo, 0u);
-                if (!EXACT && s < kUnderflow) alpha_out(std::true_type{}, i, r, xu, u, m, mui, oout, mo, muo, 0u);
-                lds_pair(yi ^ koff(r)) = make_float2(mo, muo);
-                tmax = vmax_raw(tmax, mo);
-              }
             }
           }
         }
@@ -444,20 +322,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         if (lane == 0) wmax[(k & 1) * kMaxWaves + wave] = tmax;
         rho = rho + KV >= nb ? rho + KV - nb : rho + KV;
         __syncthreads();
-      }
-
-      // kETab: the beta sweep's table replaces the alpha sweep's (every wave has
-      // left it at the last alpha step's barrier; the barriers below come before
-      // its first read): float4 entry k = (-|d|^2, sg . h, h) of LUT entry k,
-      // rows 0..15 only, its codeword written here and (e, f) per step.  A
-      // state's entry is at twice its codeword's LUT byte, its row wrapped mod 16
-      // (cbs doubled for the sweep).
-      if constexpr (kETab) {
-        float4* et = reinterpret_cast<float4*>(lut);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) et[tid + 256 * j] = make_float4(0.0f, 0.0f, hE[j][0], hE[j][1]);
-#pragma unroll
-        for (int c = 0; c < R; ++c) cbs[c] <<= 1;
       }
 
       // log2 Z and E[F] = sum_j 2^(m_{N-1}(j) - log2 Z) mu_{N-1}(j); m~ and mu of a
@@ -495,14 +359,14 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
       // Raw alpha-side inputs (m~, mu) of step t come back from HBM two
       // butterflies ahead of their use, across step boundaries.
       auto slot_src = [&](int t, int i) {
-        const int q = min(utid + i * nthr, NB - 1);
+        const int q = min(tid + i * nthr, NB - 1);
         return slot + ((size_t)t * NB + q) * 2 * R;
       };
       // The next two butterflies in consumption order (t descending, i
       // ascending).
       // A shift register of the next kSlotAhead butterflies' (m~, mu) inputs.
       float pf[kSlotAhead][R], pfu[kSlotAhead][R];
-      if constexpr (kPair) {
+      {
 #pragma unroll
         for (int d = 0; d < kSlotAhead; ++d) {
           const int tt = N - 1 - d / UPT;
@@ -529,46 +393,12 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
           nw[v] = -wbuf[t * V + v] * sk;
           sg[v] = CT::kSigma * gbuf[t * V + v];
         }
-        if constexpr (kETab) {  // every wave has left step t+1's table (barrier at its end)
-          float4* et = reinterpret_cast<float4*>(lut);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int kk = tid + 256 * j;
-            const float2 h = *reinterpret_cast<const float2*>(&et[kk].z);
-            float e = 0.0f, f = 0.0f;
-            const float d0 = fmaf(h.x, ssk, nw[0]);
-            e = fmaf(-d0, d0, e);
-            f = fmaf(sg[0], h.x, f);
-            const float d1 = fmaf(h.y, ssk, nw[1]);
-            e = fmaf(-d1, d1, e);
-            f = fmaf(sg[1], h.y, f);
-            *reinterpret_cast<float2*>(&et[kk]) = make_float2(e, f);
-          }
-          __syncthreads();
-        }
         const uint32_t yb = base_off(rho);
         uint32_t Ku[UPT], Kk[R];  // uniform per step
 #pragma unroll
         for (int i = 0; i < UPT; ++i) Ku[i] = unit_off(i, rho);
-        if constexpr (kPair) {
 #pragma unroll
-          for (int c = 0; c < R; ++c) Kk[c] = slot_off(c, rho);
-        }
-        auto koff = [&](int c) -> uint32_t {
-          if constexpr (kPair) {
-            return Kk[c];
-          } else {
-            return slot_off(c, rho);
-          }
-        };
-        // kETab: the table bases, opaque per step, so that the 16 x 16 wrapped
-        // addresses are formed where they are read, not hoisted out of the loop.
-        uint32_t cbo[kETab ? R : 1];
-        if constexpr (kETab) {
-#pragma unroll
-          for (int c = 0; c < R; ++c) cbo[c] = (uint32_t)opaque((int)cbs[c]);
-        }
-
+        for (int c = 0; c < R; ++c) Kk[c] = slot_off(c, rho);
         // Output p of butterfly u: n~ and nu of state p*NB + u from the shifted
         // inputs nr[c] (maximum 0) and raw nu inputs, and the butterfly's
         // contribution to the gradient sums (a0 for sum dll, a1 for sum dll h).
@@ -577,42 +407,9 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
                             const float (&nui)[R], float pms, float pmu, float oout, float& no, float& nuo,
                             float& a0, float (&a1)[V]) -> float {
           constexpr bool SHIFT = decltype(shift_tag)::value;
-          if constexpr (kETab && !SHIFT) {
-            // Group-sum variant (M = 0): each input's terms are summed as its
-            // table entry is read, so one entry at a time is live (the same
-            // operations as the general form below).
-            const float Dp = pmu - EFg;
-            float s = 0.0f, ez = 0.0f, ga[V];
-#pragma unroll
-            for (int c = 0; c < R; ++c) {
-              const float4 ef = *reinterpret_cast<const float4*>(smem + ((cbo[c] + 2 * hyb_col_step(p, c)) & 0x3FFFu));
-              const float e = fexp2(nr[c] + ef.x);
-              const float ezc = e * (nui[c] + ef.y);
-              s = c ? s + e : e;
-              ez = c ? ez + ezc : ezc;
-              const float wgt = fmaf(e, Dp, ezc);
-              ga[0] = c ? fmaf(wgt, ef.z, ga[0]) : wgt * ef.z;
-              ga[1] = c ? fmaf(wgt, ef.w, ga[1]) : wgt * ef.w;
-            }
-            const float G = fexp2(pms);
-            a0 = G * fmaf(Dp, s, ez);
-#pragma unroll
-            for (int v = 0; v < V; ++v) a1[v] = G * ga[v];
-            no = flog2(s) + (0.0f - oout);
-            nuo = ez * frcp(s);
-            return s;
-          }
           float y[R], z[R], hh[R][V];
 #pragma unroll
           for (int c = 0; c < R; ++c) {
-            if constexpr (kETab) {
-              const float4 ef = *reinterpret_cast<const float4*>(smem + ((cbo[c] + 2 * hyb_col_step(p, c)) & 0x3FFFu));
-              y[c] = nr[c] + ef.x;
-              z[c] = nui[c] + ef.y;
-              hh[c][0] = ef.z;
-              hh[c][1] = ef.w;
-              continue;
-            }
             if (i < CU) {
 #pragma unroll
               for (int v = 0; v < V; ++v) hh[c][v] = hcb[i < CU ? i : 0][p][c][v];
@@ -666,7 +463,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
           const uint32_t yi = yb ^ Ku[i];
 #pragma unroll
           for (int c = 0; c < R; ++c) {
-            const float2 v2 = lds_pair(yi ^ koff(c));
+            const float2 v2 = lds_pair(yi ^ Kk[c]);
             n[c] = v2.x;
             nu[c] = v2.y;
           }
@@ -679,11 +476,11 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         float tmax = -INFINITY;
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
-          const int q = utid + i * nthr;
+          const int q = tid + i * nthr;
           float pm[R], pmu[R], ni[R], nui[R];
 #pragma unroll
           for (int r = 0; r < R; ++r) {
-            if constexpr (kPair) {
+            {
               pm[r] = pf[0][r];
               pmu[r] = pfu[0][r];
 #pragma unroll
@@ -695,7 +492,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
             ni[r] = nx[r];
             nui[r] = nxu[r];
           }
-          if constexpr (kPair) {  // fetch the butterfly kSlotAhead ahead
+          {  // fetch the butterfly kSlotAhead ahead
             const int tt = t - (i + kSlotAhead) / UPT;
             const int ii = (i + kSlotAhead) % UPT;
             if (tt >= 0) {
@@ -714,7 +511,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
             const float oout = sh + Qv;
             const float kts = Kt - sh;
             const uint32_t yi = yb ^ Ku[i];
-            if constexpr (kPair) {
+            {
               float no[R], nuo[R], smin = 0.0f, ua0 = 0.0f, ua1[V];
 #pragma unroll
               for (int p = 0; p < R; ++p) {
@@ -745,62 +542,9 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
               for (int v = 0; v < V; ++v) A1[v] += ua1[v];
 #pragma unroll
               for (int p = 0; p < R; ++p) {
-                lds_pair(yi ^ koff(p)) = make_float2(no[p], nuo[p]);
+                lds_pair(yi ^ Kk[p]) = make_float2(no[p], nuo[p]);
               }
               tmax = max_with(tmax, no);
-            } else if constexpr (kColUnroll) {
-              // Outputs unrolled (immediate LUT offsets); the butterfly's gradient
-              // sums are redone when a group underflowed.
-              const float* src = slot_src(t, i);
-              float smin = 0.0f, ua0 = 0.0f, ua1[V];
-#pragma unroll
-              for (int p = 0; p < R; ++p) {
-                float no, nuo, a0, a1[V];
-                const float pms = src[2 * p] + kts, pmup = src[2 * p + 1];
-                const float s = beta_out(Fast{}, i, p, xu, u, nr, nui, pms, pmup, oout, no, nuo, a0, a1);
-                smin = p ? fminf(smin, s) : s;
-                ua0 = p ? ua0 + a0 : a0;
-#pragma unroll
-                for (int v = 0; v < V; ++v) ua1[v] = p ? ua1[v] + a1[v] : a1[v];
-                lds_pair(yi ^ koff(p)) = make_float2(no, nuo);
-                tmax = vmax_raw(tmax, no);
-              }
-              if constexpr (!EXACT) {
-                if (smin < kUnderflow) {
-                  ua0 = 0.0f;
-#pragma unroll
-                  for (int v = 0; v < V; ++v) ua1[v] = 0.0f;
-#pragma unroll 1
-                  for (int p = 0; p < R; ++p) {
-                    float no, nuo, a0, a1[V];
-                    const float pms = src[2 * p] + kts, pmup = src[2 * p + 1];
-                    beta_out(std::true_type{}, i, p, xu, u, nr, nui, pms, pmup, oout, no, nuo, a0, a1);
-                    ua0 += a0;
-#pragma unroll
-                    for (int v = 0; v < V; ++v) ua1[v] += a1[v];
-                    lds_pair(yi ^ koff(p)) = make_float2(no, nuo);
-                    tmax = vmax_raw(tmax, no);
-                  }
-                }
-              }
-              A0 += ua0;
-#pragma unroll
-              for (int v = 0; v < V; ++v) A1[v] += ua1[v];
-            } else {
-              const float* src = slot_src(t, i);
-#pragma unroll kOuterUnroll<R>
-              for (int p = 0; p < R; ++p) {
-                float no, nuo, a0, a1[V];
-                const float pms = src[2 * p] + kts, pmup = src[2 * p + 1];
-                const float s = beta_out(Fast{}, i, p, xu, u, nr, nui, pms, pmup, oout, no, nuo, a0, a1);
-                if (!EXACT && s < kUnderflow)
-                  beta_out(std::true_type{}, i, p, xu, u, nr, nui, pms, pmup, oout, no, nuo, a0, a1);
-                A0 += a0;
-#pragma unroll
-                for (int v = 0; v < V; ++v) A1[v] += a1[v];
-                lds_pair(yi ^ koff(p)) = make_float2(no, nuo);
-                tmax = vmax_raw(tmax, no);
-              }
             }
           }
         }
@@ -816,10 +560,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         if (lane == 0) wmax[(k & 1) * kMaxWaves + wave] = tmax;
         rho = rho - KV < 0 ? rho - KV + nb : rho - KV;
         __syncthreads();
-      }
-      if constexpr (kETab) {  // the alpha sweep's undoubled bases
-#pragma unroll
-        for (int c = 0; c < R; ++c) cbs[c] >>= 1;
       }
     };
     if (Tb < kExactBelowT) {
@@ -854,13 +594,6 @@ const void* bwd_kernel_ptr(int KV, int V, int code, int upt) {
   BCJR_BWD_UPTS(2, 1, CODE_3INST)
   BCJR_BWD_UPTS(2, 2, CODE_TABLE)
   BCJR_BWD_UPTS(2, 2, CODE_HYB)
-  // kV = 4: whole 16-state butterflies, at most 256 per sequence (L <= 16).
-  BCJR_BWD_CASE(4, 1, CODE_TABLE, 1)
-  BCJR_BWD_CASE(4, 1, CODE_1MAD, 1)
-  BCJR_BWD_CASE(4, 1, CODE_3INST, 1)
-  BCJR_BWD_CASE(4, 2, CODE_TABLE, 1)
-  BCJR_BWD_CASE(4, 2, CODE_HYB, 1)
-  BCJR_BWD_CASE(4, 2, CODE_HYB_COL, 1)
   return nullptr;
 }
 

@@ -73,6 +73,7 @@ struct Plan {
   const void* fn = nullptr;
   size_t lds = 0;
   size_t slot_bytes = 0;
+  int num_cu = 0;
   int max_blocks = 0;  // resident blocks on the device
   bcjr::Swizzle swz = {{31, 31, 31, 31}, {0, 0, 0, 0}};
 };
@@ -106,7 +107,13 @@ int validate(const bcjr_problem* p) {
   return BCJR_OK;
 }
 
-enum { OP_FWD = BCJR_OP_FORWARD, OP_BWD = BCJR_OP_BACKWARD, OP_VIT = BCJR_OP_VITERBI, OP_FWD_INTERNALS = 3 };
+enum {
+  OP_FWD = BCJR_OP_FORWARD,
+  OP_BWD = BCJR_OP_BACKWARD,
+  OP_VIT = BCJR_OP_VITERBI,
+  OP_FWD_INTERNALS = 3,
+  OP_FWD_ENTROPY = 4
+};
 
 // Bytes of one sequence slot of an operation's workspace (a validated problem):
 // forward N * 2^(L-kV) floats (the raw alpha inputs of every step), backward
@@ -139,11 +146,11 @@ int check_ws(const bcjr_problem* p, int op, const void* ws, size_t ws_bytes) {
 // steady-state calls (and calls made while a stream is being captured into a
 // graph) do no attribute or occupancy queries.
 struct PlanKey {
-  int dev, op, L, k, V, code, Q;
+  int dev, op, L, k, V, code, Q, wide;
   long long N;
   bool operator==(const PlanKey& o) const {
     return dev == o.dev && op == o.op && L == o.L && k == o.k && V == o.V && code == o.code &&
-           Q == o.Q && N == o.N;
+           Q == o.Q && wide == o.wide && N == o.N;
   }
 };
 constexpr int kPlanCache = 64;
@@ -152,15 +159,17 @@ PlanKey g_plan_keys[kPlanCache];
 Plan g_plans[kPlanCache];
 int g_plan_count = 0, g_plan_next = 0;
 
-int make_plan_uncached(const bcjr_problem* p, int op, const DeviceInfo& di, Plan* pl);
+int make_plan_uncached(const bcjr_problem* p, int op, bool wide, const DeviceInfo& di, Plan* pl);
 
-int make_plan(const bcjr_problem* p, int op, Plan* pl) {
+// wide: the launch shape of a batch too small to fill the chip, where the
+// operation has one of its own (make_soft16_plan), else the same plan.
+int make_plan(const bcjr_problem* p, int op, Plan* pl, bool wide = false) {
   int rc = validate(p);
   if (rc) return rc;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-  const PlanKey key = {dev, op, p->L, p->k, p->V, p->code, p->code == BCJR_CODE_HYB ? p->Q : 0,
+  const PlanKey key = {dev, op, p->L, p->k, p->V, p->code, p->code == BCJR_CODE_HYB ? p->Q : 0, wide ? 1 : 0,
                        (long long)p->N};
   {
     std::lock_guard<std::mutex> lk(g_plan_mu);
@@ -173,7 +182,7 @@ int make_plan(const bcjr_problem* p, int op, Plan* pl) {
   DeviceInfo di;
   rc = device_info(&di);
   if (rc) return rc;
-  rc = make_plan_uncached(p, op, di, pl);
+  rc = make_plan_uncached(p, op, wide, di, pl);
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(g_plan_mu);
   const int slot = g_plan_count < kPlanCache ? g_plan_count++ : (g_plan_next++ % kPlanCache);
@@ -271,8 +280,51 @@ bcjr::Swizzle pick_swizzle(int L, int KV) {
 // slots and the rotations 0, 4, 8 (the search above assumes u = tid).
 constexpr bcjr::Swizzle kColWalkSwizzle = {{4, 6, 8, 31}, {3u, 31u, 15u, 0u}};
 
-int make_plan_uncached(const bcjr_problem* p, int op, const DeviceInfo& di, Plan* pl) {
+// Opts the plan's kernel in to its LDS and finds how many blocks the device holds.
+int finish_plan(const bcjr_problem* p, const DeviceInfo& di, Plan* pl) {
+  if (pl->lds > di.max_lds)
+    return fail(BCJR_EUNSUPPORTED, "needs %zu bytes of LDS per workgroup (device limit %zu); reduce N=%lld",
+                pl->lds, di.max_lds, (long long)p->N);
+  hipError_t e = hipFuncSetAttribute(pl->fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->lds);
+  if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
+  int per_cu = 0;
+  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pl->fn, pl->nthr, pl->lds);
+  if (e != hipSuccess) return hip_fail(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+  if (per_cu < 1)
+    return fail(BCJR_EUNSUPPORTED, "kernel cannot be resident (%d threads, %zu B LDS)", pl->nthr, pl->lds);
+  pl->num_cu = di.num_cu;
+  pl->max_blocks = per_cu * di.num_cu;
+  return BCJR_OK;
+}
+
+// The soft kernels of 4-bit steps (bcjr_soft16.h).  Lanes per butterfly: the
+// column walk 2 (512 threads, two workgroups per CU), or 4 (1,024 threads) where
+// the workgroup has its CU to itself anyway (wide); other codes 4, and 16 for the
+// NB <= 32 butterflies of L <= 13, which 4 would leave on one or two waves.
+int make_soft16_plan(const bcjr_problem* p, int op, bool wide, const DeviceInfo& di, Plan* pl) {
+  const int code = bcjr::soft_kernel_code(p->code, p->L, 4, p->Q);
+  const int kind = op == OP_BWD ? 1 : op == OP_FWD_ENTROPY ? 2 : 0;
+  const int lpb = code == bcjr::CODE_HYB_COL ? (wide ? 4 : 2) : p->L <= 13 ? 16 : 4;
+  pl->KV = 4;
+  pl->R = 16;
+  pl->NSUB = 1;
+  pl->NT = 1 << (p->L - 4);
+  pl->NB = pl->NT >> 4;
+  pl->NU = pl->NB;
+  pl->upt = 1;
+  const int per_wave = 64 / lpb;  // butterflies of a wave
+  pl->nthr = (pl->NB + per_wave - 1) / per_wave * 64;
+  pl->fn = bcjr::soft16_kernel_ptr(kind, p->V, code, lpb);
+  pl->lds = bcjr::soft16_lds_bytes(p->L, p->V, (int)p->N, pl->nthr / 64, code, p->Q, kind);
+  pl->swz = code == bcjr::CODE_HYB_COL ? kColWalkSwizzle : pick_swizzle(p->L, 4);
+  pl->slot_bytes = slot_bytes_of(p, op == OP_BWD ? OP_BWD : OP_FWD);
+  return finish_plan(p, di, pl);
+}
+
+int make_plan_uncached(const bcjr_problem* p, int op, bool wide, const DeviceInfo& di, Plan* pl) {
   const int KV = p->k * p->V, R = 1 << KV, RO = R < 4 ? R : 4;
+  if (KV == 4 && (op == OP_FWD || op == OP_BWD || op == OP_FWD_ENTROPY)) return make_soft16_plan(p, op, wide, di, pl);
+  if (op == OP_FWD_ENTROPY) op = OP_FWD_INTERNALS;
   pl->KV = KV;
   pl->R = R;
   pl->NSUB = R / RO;
@@ -338,7 +390,7 @@ int make_plan_uncached(const bcjr_problem* p, int op, const DeviceInfo& di, Plan
     pl->slot_bytes = slot_bytes_of(p, fwd ? OP_FWD : OP_VIT);
   } else {
     pl->cache = false;
-    pl->swz = kcode == bcjr::CODE_HYB_COL ? kColWalkSwizzle : pick_swizzle(p->L, KV);
+    pl->swz = pick_swizzle(p->L, KV);
     pl->fn = bcjr::bwd_kernel_ptr(KV, p->V, kcode, upt);
     pl->lds = bcjr::bwd_lds_bytes(p->L, KV, p->V, N, nwaves, kcode, p->Q);
     pl->slot_bytes = slot_bytes_of(p, OP_BWD);
@@ -346,17 +398,7 @@ int make_plan_uncached(const bcjr_problem* p, int op, const DeviceInfo& di, Plan
   if (!pl->fn)
     return fail(BCJR_EUNSUPPORTED, "no kernel built for L=%d k=%d V=%d code=%d (units/thread %d)",
                 p->L, p->k, p->V, p->code, upt);
-  if (pl->lds > di.max_lds)
-    return fail(BCJR_EUNSUPPORTED, "needs %zu bytes of LDS per workgroup (device limit %zu); reduce N=%lld",
-                pl->lds, di.max_lds, (long long)p->N);
-  hipError_t e = hipFuncSetAttribute(pl->fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->lds);
-  if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
-  int per_cu = 0;
-  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pl->fn, nthr, pl->lds);
-  if (e != hipSuccess) return hip_fail(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-  if (per_cu < 1) return fail(BCJR_EUNSUPPORTED, "kernel cannot be resident (%d threads, %zu B LDS)", nthr, pl->lds);
-  pl->max_blocks = per_cu * di.num_cu;
-  return BCJR_OK;
+  return finish_plan(p, di, pl);
 }
 
 int launch(const Plan& pl, long long B, size_t ws_bytes, void* params, hipStream_t stream) {
@@ -375,6 +417,100 @@ int launch(const Plan& pl, long long B, size_t ws_bytes, void* params, hipStream
 }
 
 }  // namespace
+
+size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Bytes the two-halves launches keep per sequence: its slot, the two state
+// vectors where the sweeps meet, and the offsets of every step.
+size_t halves_bytes(const bcjr_problem* p, int op) {
+  const size_t NT = (size_t)1 << (p->L - p->k * p->V), st = op == OP_BWD ? 2 : 1;
+  return slot_bytes_of(p, op == OP_BWD ? OP_BWD : OP_FWD) + round256(2 * st * NT * sizeof(float)) +
+         round256(((size_t)p->N + 2) * sizeof(double));
+}
+
+// Whether a kV = 4 soft call runs its sequences in two halves each (bcjr_soft16.h),
+// on which plan: when twice as many workgroups still all fit at once, so that
+// the steps in sequence are halved and no sequence waits for another.  The choice
+// depends on the problem and the device only, not on the workspace (a short one
+// takes several rounds), so every workspace gives the same bits.  Column walk:
+// one workgroup of twice the threads per CU where that is all there is.
+// MEASURED16
+int halves_plan(const bcjr_problem* p, int op, const Plan& pl, Plan* out, bool* halves) {
+  *halves = p->N >= 2 && 2 * p->B <= pl.max_blocks;
+  *out = pl;
+  if (*halves && bcjr::soft_kernel_code(p->code, p->L, 4, p->Q) == bcjr::CODE_HYB_COL && 2 * p->B <= pl.num_cu)
+    return make_plan(p, op, out, true);
+  return BCJR_OK;
+}
+
+// Bytes of the transposed codebook copy of the kV = 4 table kernels (0: none).
+size_t table16_bytes(const bcjr_problem* p) {
+  return p->k * p->V == 4 && p->code == BCJR_CODE_TABLE ? round256(((size_t)p->V << p->L) * sizeof(float)) : 0;
+}
+
+// One kV = 4 soft call: the table's transposed copy (when the workspace has room
+// for it beside one slot; else the kernels read the table as it is), then the
+// batch in two halves or in one launch.
+int launch_soft16(const bcjr_problem* p, int op, bcjr::Soft16Params P, void* ws, size_t ws_bytes,
+                  hipStream_t stream) {
+  Plan pl, hp;
+  int rc = make_plan(p, op, &pl);
+  if (rc) return rc;
+  bool halves = false;
+  rc = halves_plan(p, op, pl, &hp, &halves);
+  if (rc) return rc;
+  char* w = static_cast<char*>(ws);
+  size_t left = ws_bytes;
+  P.SC = 1;
+  P.SU = 16;
+  const size_t tb = table16_bytes(p);
+  if (tb && left >= tb + pl.slot_bytes) {
+    hipError_t e = bcjr::launch_transpose16(P.table, reinterpret_cast<float*>(w), p->L, p->V, stream);
+    if (e != hipSuccess) return hip_fail(e, "codebook transpose launch");
+    P.table = reinterpret_cast<const float*>(w);
+    P.SC = (uint32_t)pl.NB;
+    P.SU = 1;
+    w += tb;
+    left -= tb;
+  }
+  P.N = (int)p->N;
+  P.L = p->L;
+  P.Q = p->Q;
+  P.t_per_seq = p->t_per_seq ? 1 : 0;
+  P.swz = pl.swz;
+  P.ws = reinterpret_cast<float*>(w);
+  P.slot_floats = pl.slot_bytes / sizeof(float);
+  const size_t per = halves_bytes(p, op);
+  const long long round = halves ? std::min<long long>(p->B, (long long)(left / per)) : 0;
+  if (round < 1) {
+    P.mode = 0;
+    P.B = p->B;
+    return launch(pl, p->B, left, &P, stream);
+  }
+  const size_t NT = (size_t)pl.NT, st = op == OP_BWD ? 2 : 1, row = (size_t)p->N * p->V;
+  char* mid = w + (size_t)round * pl.slot_bytes;
+  P.mid = reinterpret_cast<float*>(mid);
+  P.moff = reinterpret_cast<double*>(mid + (size_t)round * round256(2 * st * NT * sizeof(float)));
+  for (long long b0 = 0; b0 < p->B; b0 += round) {
+    bcjr::Soft16Params H = P;
+    H.B = std::min<long long>(round, p->B - b0);
+    H.seq += b0 * row;
+    H.out += b0 * row;
+    if (P.t_per_seq) H.T += b0;
+    if (H.logZ) H.logZ += b0;
+    if (H.H_out) H.H_out += b0 * p->N;
+    if (H.g_soft) H.g_soft += b0 * row;
+    if (H.g_logZ) H.g_logZ += b0;
+    for (H.mode = 1; H.mode <= 2; ++H.mode) {
+      void* args[] = {&H};
+      hipError_t e = hipLaunchKernel(hp.fn, dim3((unsigned)(2 * H.B)), dim3((unsigned)hp.nthr), args, hp.lds, stream);
+      if (e != hipSuccess) return hip_fail(e, "hipLaunchKernel");
+      e = hipGetLastError();
+      if (e != hipSuccess) return hip_fail(e, "kernel launch");
+    }
+  }
+  return BCJR_OK;
+}
 
 // Sequence slots of bcjr_forward_noalloc: a static device array, one copy per
 // GPU.  Host code never names it after set-up: its host-side symbol is only a
@@ -454,6 +590,14 @@ int bcjr_workspace_bytes(const bcjr_problem* prob, int op, size_t* bytes) {
   if (rc) return rc;
   const long long slots = std::max<long long>(1, std::min<long long>(prob->B, pl.max_blocks));
   *bytes = (size_t)slots * pl.slot_bytes;
+  if (pl.KV == 4 && op != OP_VIT) {
+    Plan hp;
+    bool halves = false;
+    rc = halves_plan(prob, op, pl, &hp, &halves);
+    if (rc) return rc;
+    if (halves) *bytes = std::max(*bytes, (size_t)prob->B * halves_bytes(prob, op));
+    *bytes += table16_bytes(prob);
+  }
   return BCJR_OK;
 }
 
@@ -464,6 +608,15 @@ int bcjr_forward(const bcjr_problem* prob, const float* seq, const float* T, con
   if (!seq || !T || !soft || !ws) return fail(BCJR_EINVAL, "seq, T, soft and ws must be non-NULL");
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
+  if (prob->k * prob->V == 4) {
+    bcjr::Soft16Params S = {};
+    S.seq = seq;
+    S.T = T;
+    S.table = codebook_or_lut;
+    S.out = soft;
+    S.logZ = logZ;
+    return launch_soft16(prob, OP_FWD, S, ws, ws_bytes, stream);
+  }
   Plan pl;
   int rc = make_plan(prob, OP_FWD, &pl);
   if (rc) return rc;
@@ -536,8 +689,18 @@ int bcjr_forward_entropy(const bcjr_problem* prob, const float* seq, const float
     return fail(BCJR_EINVAL, "seq, T, soft, ws and entropy must be non-NULL");
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
+  if (prob->k * prob->V == 4) {
+    bcjr::Soft16Params S = {};
+    S.seq = seq;
+    S.T = T;
+    S.table = codebook_or_lut;
+    S.out = soft;
+    S.logZ = logZ;
+    S.H_out = entropy;
+    return launch_soft16(prob, OP_FWD_ENTROPY, S, ws, ws_bytes, stream);
+  }
   Plan pl;
-  int rc = make_plan(prob, OP_FWD_INTERNALS, &pl);
+  int rc = make_plan(prob, OP_FWD_ENTROPY, &pl);
   if (rc) return rc;
   bcjr::FwdParams P = {};
   P.seq = seq;
@@ -565,6 +728,16 @@ int bcjr_backward(const bcjr_problem* prob, const float* seq, const float* T, co
     return fail(BCJR_EINVAL, "seq, T, g_soft, g_seq and ws must be non-NULL");
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
+  if (prob->k * prob->V == 4) {
+    bcjr::Soft16Params S = {};
+    S.seq = seq;
+    S.T = T;
+    S.table = codebook_or_lut;
+    S.out = g_seq;
+    S.g_soft = g_soft;
+    S.g_logZ = g_logZ;
+    return launch_soft16(prob, OP_BWD, S, ws, ws_bytes, stream);
+  }
   Plan pl;
   int rc = make_plan(prob, OP_BWD, &pl);
   if (rc) return rc;

@@ -28,7 +28,7 @@
 namespace bcjr {
 
 // CODE_HYB_COL is HYB with its LUT staged for the column walk (hyb_col_base);
-// the soft kernels take it at L = 16, kV = 4, 3 <= Q <= 9.  It never crosses the
+// the soft and Viterbi kernels take it at L = 16, kV = 4, 3 <= Q <= 9.  It never crosses the
 // C ABI.
 enum { CODE_TABLE = 0, CODE_1MAD = 1, CODE_3INST = 2, CODE_HYB = 3, CODE_HYB_COL = 4 };
 
@@ -118,17 +118,27 @@ __device__ __forceinline__ uint32_t hyb_col_step(int p, int r) {
   return ((uint32_t)(p * (2 * r + 1)) & 15u) << 9;
 }
 
+// The states of p and p + 8 sit 8 rows apart (8 (2r + 1) mod 16 = 8), and rows 8
+// apart hold the same LUT entry with the sign of its second component flipped.
+// A 16-byte table entry for both (codeword, own emission, emission 8 rows on)
+// at hyb_col_base doubled + hyb_pair_step(p, r), p < 8, therefore serves the two
+// states: it is the entry of p (and, 8 rows on, of p + 8), or with hyb_pair_far
+// that of p + 8.  base + step spans rows 0 .. 22 of 1,024 bytes.
+__host__ __device__ constexpr uint32_t hyb_pair_step(int p, int r) {
+  return ((uint32_t)(p * (2 * r + 1)) & 7u) << 10;
+}
+__host__ __device__ constexpr bool hyb_pair_far(int p, int r) { return ((p * (2 * r + 1)) & 8) != 0; }
+
 __device__ __forceinline__ float2 hyb_col_read(const unsigned char* lutb, uint32_t off) {
   return *reinterpret_cast<const float2*>(lutb + off);
 }
 
-// Butterfly of thread tid in the column-walk soft kernels (256 threads, one
-// 16-state butterfly each).  The LUT column of state 16u + c is bits [6, 12) of
-// x = s^2 + s for Q = 9 (the reference's LUT).  Over each coset of span(bits
-// 2..7 of u) those columns are all 64 distinct, for every c, so a wave owns one
-// coset: u takes tid's bits 0..5 as its bits 2..7 and the wave index as its bits
-// 0, 1.  Then a half-wave's 8-byte LUT reads hit 32 distinct banks and a wave's
-// 4-byte reads of a per-step table in the LUT's layout 64 distinct banks
+// Butterfly of lane slot q (0..255) in the column-walk soft kernel (LPB lanes of a
+// wave share the 64 / LPB consecutive slots of the wave).  The LUT column of
+// state 16u + c is bits [6, 12) of x = s^2 + s for Q = 9 (the reference's LUT).
+// Over each coset of span(bits 2..7 of u) those columns are all 64 distinct, for
+// every c, so 64 slots own one coset: u takes q's bits 0..5 as its bits 2..7 and
+// q >> 6 as its bits 0, 1.  Then 32 slots' table reads hit distinct banks
 // (checked in tests/test_capi_cpu.py).  (A smaller Q has fewer columns.)
 __host__ __device__ constexpr uint32_t col_walk_unit(uint32_t tid) {
   return ((tid >> 6) & 3u) | ((tid & 63u) << 2);
@@ -136,20 +146,12 @@ __host__ __device__ constexpr uint32_t col_walk_unit(uint32_t tid) {
 
 // LDS layout of the column-walk forward's one state vector: with the rotation of
 // step t applied, x = rotr(j, rho_t), reduced state j sits at element
-// col_walk_state_el(x).  Under col_walk_unit, every 32-bit read (64 lanes, banks
-// mod 64) and write (32 lanes, mod 32) of x = rotr(k*256 + u, rho) is
-// conflict-free, for k < 16 and rho = 0, 4, 8.  Linear, so the element of
-// k*256 + u is that of u XOR that of k*256.
+// col_walk_state_el(x).  Under col_walk_unit, every 32-bit access of 64 (reads,
+// banks mod 64) or 32 (writes, mod 32) slots to x = rotr(k*256 + u, rho) is
+// conflict-free, for k < 16 and rho = 0, 4, 8; lanes that share a butterfly read
+// the same words.  Linear, so the element of k*256 + u is that of u XOR that of k*256.
 __host__ __device__ constexpr uint32_t col_walk_state_el(uint32_t x) {
   return x ^ ((x >> 4) & 3u) ^ ((x >> 6) & 63u) ^ ((x >> 7) & 31u);
-}
-
-// Any state from the column-walk LUT (rows 0..15).
-__device__ __forceinline__ void code_hyb_col(uint32_t s, const float2* lut2c, int Q, float& c0, float& c1) {
-  const uint32_t x = __umul24(s, s) + s;
-  const float2 v = lut2c[(((x >> 12) & 15u) << 6) | ((x >> (15 - Q)) & ((1u << (Q - 3)) - 1u))];
-  c0 = v.x;
-  c1 = v.y;
 }
 
 // Fills the column-walk LUT from the (2^Q, 2) table: entry (row, col) is signed
@@ -266,8 +268,6 @@ __device__ __forceinline__ void raw_codeword(uint32_t xu, uint32_t off, uint32_t
   } else if constexpr (CODE == CODE_TABLE) {
 #pragma unroll
     for (int v = 0; v < V; ++v) h[v] = table[(size_t)s * V + v];
-  } else if constexpr (CODE == CODE_HYB_COL) {
-    code_hyb_col(s, reinterpret_cast<const float2*>(lut), Q, h[0], h[1]);
   } else {
     code_hyb_signed(s, reinterpret_cast<const float2*>(lut), Q, h[0], h[1]);
   }
@@ -537,6 +537,26 @@ struct BwdParams {
   long long B;
   int N, L, Q, t_per_seq;
   Swizzle swz;          // LDS layout of (m~, mu) and (n~, nu)
+};
+
+// The kV = 4 soft kernels (bcjr_soft16.h).
+struct Soft16Params {
+  const float* seq;      // (B, N, V)
+  const float* T;        // (B,) or (1,)
+  const float* table;    // codebook (any of the two layouts of SC, SU) or (2^Q, 2) LUT
+  float* out;            // (B, N, V) soft codeword, or d seq of the backward
+  float* logZ;           // (B,) or null
+  float* H_out;          // (B, N) marginal entropy in nats (entropy instances)
+  const float* g_soft;   // (B, N, V), backward
+  const float* g_logZ;   // (B,) or null, backward
+  float* ws;             // slots of slot_floats floats: raw inputs of every step
+  float* mid;            // two halves: (B, 2, NT) state vectors (backward: pairs) where the sweeps meet
+  double* moff;          // two halves: (B, N + 2) offsets of the stored inputs, then of the two vectors
+  size_t slot_floats;
+  long long B;
+  int N, L, Q, t_per_seq, mode;
+  uint32_t SC, SU;       // table strides (bcjr_soft16.h)
+  Swizzle swz;           // LDS layout of the state vector
 };
 
 struct VitParams {

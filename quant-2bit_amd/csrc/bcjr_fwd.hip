@@ -1,4 +1,6 @@
-// Soft forward pass of the BCJR node: soft codewords E_P[c(s_t)] and log Z.
+// Soft forward pass of the BCJR node: soft codewords E_P[c(s_t)] and log Z, for
+// kV <= 2, and the diagnostics forward for every kV (bcjr_soft16.h runs the plain
+// kV = 4 forward).
 //
 // Replaces the compute of bcjr_forward_backward (src/bcjr/forward_backward.py:190-232)
 // and the forward of BcjrForwardBackwardMonolithic (src/bcjr/bcjr_monolithic.py:161-189).
@@ -41,22 +43,17 @@
 namespace bcjr {
 
 template <int KV, int V, int CODE, int UPT, int CU, bool INTERNALS>
-__global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_COL && !INTERNALS ? 3 : 1) void bcjr_fwd_kernel(
-    FwdParams P) {
+__global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, 1) void bcjr_fwd_kernel(FwdParams P) {
   constexpr int R = 1 << KV;
   // Butterflies of 2 or 4 states run fully unrolled with their slot inputs
-  // prefetched in registers; 16-state butterflies loop over outputs (unrolled
-  // too on the HYB column walk, whose LUT offsets are then immediates).
+  // prefetched in registers; 16-state butterflies (diagnostics only) loop over
+  // outputs.
   constexpr bool kPair = R <= 4;
   static_assert(CU == 0 || kPair, "codeword cache is for butterflies of at most 4 states");
   static_assert(CU <= UPT, "at most UPT cached butterflies");
   constexpr bool kCol = CODE == CODE_HYB_COL;  // HYB column walk: one butterfly per thread
   static_assert(!kCol || (KV == 4 && UPT == 1), "the column walk is for L = 16, kV = 4");
-  // Its outputs are unrolled except in the diagnostics instance, which would spill.
-  constexpr bool kColUnroll = kCol && !INTERNALS;
-  // Its sweeps read each state's emission (and, in the beta sweep, codeword)
-  // from a per-step table, and keep one state vector, updated in place (below).
-  constexpr bool kETab = kColUnroll;
+  static_assert(kPair || INTERNALS, "the plain kV = 4 forward is bcjr_soft16_kernel");
   using CT = CodeTraits<CODE>;
 
   extern __shared__ __align__(16) unsigned char smem[];
@@ -66,21 +63,10 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
   const uint32_t ANT = opaque_uniform(CT::A * (uint32_t)NT);  // hash offset of p * NT
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int lane = tid & 63, wave = tid >> 6, nwaves = nthr >> 6;
-  // The column-walk instance gives thread tid butterfly col_walk_unit(tid), so
-  // that its table reads hit distinct banks; elsewhere u = tid.
-  const int utid = kColUnroll ? (int)col_walk_unit((uint32_t)tid) : tid;
-  // kETab: the one state vector is updated in place.  At step t (either sweep)
-  // butterfly u reads and writes the elements st_el(k*NB + u, rho_t), k < R,
-  // rho_t = kV (t - 1) mod nb: rotr(R*u + r, kV) = r*NB + u, so its outputs land
-  // on its inputs, and col_walk_state_el keeps every access conflict-free.
-  const int nbits = L - KV;
-  auto st_el = [&](uint32_t j, int rho) -> uint32_t { return col_walk_state_el(rotr_bits(j, rho, nbits)); };
-
   double* cvec = reinterpret_cast<double*>(smem);                // N    C_{t-1}
-  // Reduced state (16-B aligned): 2*NT floats, double-buffered by step; kETab:
-  // NT floats, then the 32 KiB table region.
+  // Reduced state (16-B aligned): 2*NT floats, double-buffered by step.
   float* mbuf = reinterpret_cast<float*>(cvec + ((N + 1) & ~1));
-  float* wmax = mbuf + (kETab ? NT + 8192 : 2 * NT);              // 2*kMaxWaves
+  float* wmax = mbuf + 2 * NT;                                    // 2*kMaxWaves
   float* wsum = wmax + 2 * kMaxWaves;                             // kMaxWaves
   // Last wsum word: the block-wide input flag (at most 8 waves use wsum, launch
   // bounds 512 threads), 0 outside the check at the start of each sequence.
@@ -91,46 +77,22 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
   constexpr int SP = V + 1;
   float* spart = wbuf + N * V;                                    // 2*nwaves*SP per-wave partials
   // HYB: signed LUT (code_hyb_signed) or column-walk LUT (hyb_col_base), 8-byte
-  // aligned; kETab: the per-step tables after the state vector, 16-byte aligned.
-  float* lut = kETab ? mbuf + NT
-                     : reinterpret_cast<float*>(smem) +
-                           ((spart + 2 * nwaves * SP - reinterpret_cast<float*>(smem) + 1) & ~1);
+  // aligned.
+  float* lut = reinterpret_cast<float*>(smem) + ((spart + 2 * nwaves * SP - reinterpret_cast<float*>(smem) + 1) & ~1);
 
   if constexpr (CODE == CODE_HYB) {
     stage_hyb_signed(reinterpret_cast<float2*>(lut), P.table, P.Q, tid, nthr);
     __syncthreads();
-  } else if constexpr (kCol && !kETab) {
+  } else if constexpr (kCol) {
     stage_hyb_col(reinterpret_cast<float2*>(lut), P.table, P.Q, tid, nthr);
     __syncthreads();
   }
   const unsigned char* lutb = reinterpret_cast<const unsigned char*>(lut);
-  float2* hcomp = reinterpret_cast<float2*>(lut + 4096);  // kETab, alpha sweep
-  // Per-step tables of the column walk, in the 32 KiB region.  Alpha sweep:
-  // float k of the table (the column-walk layout: 32 rows of 64, rows 16..31
-  // repeating 0..15) holds the emission -|d|^2 of LUT entry k, d = c sk - w_t sk;
-  // two tables, for the step parities, take 16 KiB.  State s's emission sits at
-  // a quarter of the byte its codeword would have in a float4 table (plus 8 KiB
-  // for odd steps), and a wave's 64 reads fall in distinct banks (col_walk_unit).
-  // Beta sweep: one float4 table, entry k = (c, -|d|^2, 0) of LUT entry k, whose
-  // emissions are rewritten per step behind a barrier.  The kernel runs 256
-  // threads here; thread tid forms entries tid + 256j (j < 4) and their row
-  // copies.  The codewords come from the LDS: during the alpha sweep from a
-  // float2 copy of LUT entries 0..1023 in the region's second half (hcomp,
-  // filled per sequence from the (2^Q, 2) table as stage_hyb_col forms them),
-  // during the beta sweep from the float4 table itself.
-  auto col_codeword = [&](int kk, float& h0, float& h1) {
-    const int ncol = 1 << (P.Q - 3), mask = (1 << P.Q) - 1;
-    const int col = kk & 63, ii = col + ncol * (kk >> 6), ie = ii & mask;
-    h0 = col < ncol ? P.table[2 * ie] : 0.0f;
-    const float y = col < ncol ? P.table[2 * ie + 1] : 0.0f;
-    h1 = (ii >> P.Q) ? -y : y;
-  };
-  // Column-walk bases of this thread's butterfly u = utid, input c (state R*u + c)
-  // (kETab: doubled, the float4 table's byte of the row 0 entry).
+  // Column-walk bases of this thread's butterfly u = tid, input c (state R*u + c).
   uint32_t cbs[kCol ? R : 1];
   if constexpr (kCol) {
 #pragma unroll
-    for (int c = 0; c < R; ++c) cbs[c] = hyb_col_base((uint32_t)(R * min(utid, NB - 1) + c), P.Q) << (kETab ? 1 : 0);
+    for (int c = 0; c < R; ++c) cbs[c] = hyb_col_base((uint32_t)(R * min(tid, NB - 1) + c), P.Q);
   }
 
   // Raw codewords h of this thread's first CU butterflies, fixed for the
@@ -139,7 +101,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
   if constexpr (CU > 0) {
 #pragma unroll
     for (int i = 0; i < CU; ++i) {
-      const int u = min(utid + i * nthr, NB - 1);
+      const int u = min(tid + i * nthr, NB - 1);
       const uint32_t xu = CT::A * (uint32_t)(R * u) + CT::B;
 #pragma unroll
       for (int p = 0; p < R; ++p)
@@ -185,15 +147,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
       bad |= !__builtin_isfinite(w);
     }
     // m~_{-1} = log2(R) everywhere: the buffer step 0 reads from.
-    for (int j = tid; j < NT; j += nthr) mbuf[(kETab ? 0 : NT) + j] = (float)KV;
-    if constexpr (kETab) {  // the previous sequence's last barrier ended every table read
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float h0, h1;
-        col_codeword(tid + 256 * j, h0, h1);
-        hcomp[tid + 256 * j] = make_float2(h0, h1);
-      }
-    }
+    for (int j = tid; j < NT; j += nthr) mbuf[NT + j] = (float)KV;
     if (tid < 2 * kMaxWaves) wmax[tid] = -INFINITY;  // waves that do not exist
     if (bad) *bflag = 1;
     __syncthreads();
@@ -227,40 +181,11 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
       using Fast = std::integral_constant<bool, EXACT>;
 
       // ------------------------------ alpha sweep ------------------------------
-      // Emission table of step t into table t & 1 (kETab).
-      auto build_etab = [&](int t) {
-        float nwt[V];
-#pragma unroll
-        for (int v = 0; v < V; ++v) nwt[v] = -wbuf[t * V + v] * sk;
-        float* et = lut + 2048 * (t & 1);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float2 h = hcomp[tid + 256 * j];
-          const float d0 = fmaf(h.x, ssk, nwt[0]);
-          const float d1 = fmaf(h.y, ssk, nwt[1]);
-          const float e = fmaf(-d1, d1, fmaf(-d0, d0, 0.0f));
-          const int k = tid + 256 * j;
-          et[k] = e;
-          et[k + 1024] = e;
-        }
-      };
-      if constexpr (kETab) {
-        build_etab(0);
-        __syncthreads();
-      }
       double C = 0.0;  // C_{t-1}
       int k = 0;       // step counter across both sweeps: LDS buffer / wmax parity
-      int rho = nbits - KV;  // kV (t - 1) mod nb at t = 0 (kETab)
       for (int t = 0; t < N; ++t, ++k) {
-        const float* prev = mbuf + (kETab ? 0 : ((k + 1) & 1) * NT);
-        float* cur = mbuf + (kETab ? 0 : (k & 1) * NT);
-        // kETab: element st_el(k*NB + u, rho) = ebase ^ Kel[k] of butterfly u = utid
-        const uint32_t ebase = kETab ? st_el((uint32_t)utid, rho) : 0u;
-        uint32_t Kel[kETab ? R : 1];
-        if constexpr (kETab) {
-#pragma unroll
-          for (int q = 0; q < R; ++q) Kel[q] = st_el((uint32_t)(q * NB), rho);
-        }
+        const float* prev = mbuf + ((k + 1) & 1) * NT;
+        float* cur = mbuf + (k & 1) * NT;
         float O = (float)KV;  // m~_{-1} = log2(R) for every j
         if (t > 0) {
           O = -INFINITY;
@@ -271,11 +196,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         float nw[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) nw[v] = -wbuf[t * V + v] * sk;
-        // The next step's emission table goes where step t - 1's was, which
-        // every wave has left (barrier at the end of each step).
-        if (kETab && t + 1 < N) build_etab(t + 1);
-        const uint32_t eoff = 8192u * (uint32_t)(t & 1);
-
         // Output r of butterfly u (unit i) from the shifted inputs m[p]
         // (maximum 0): returns the group sum, mo = m~_t(R*u + r).
         // cb: the column-walk base of state R*u + r (kCol only).
@@ -289,9 +209,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
             // The two-rounding d_3inst form is kept out of the low-temperature
             // variant, where |d| reaches ~1e2 and float32 precision is tightest.
             const bool cached = i < CU;
-            if constexpr (kETab) {  // cb: the table byte of state R*u + r's row 0 entry
-              acc += *reinterpret_cast<const float*>(lutb + cb + (hyb_col_step(p, r) >> 1));
-            } else if (!cached && CODE == CODE_3INST && !EXACT) {
+            if (!cached && CODE == CODE_3INST && !EXACT) {
               const float d = d_3inst(xu + p * ANT + CT::A * (uint32_t)r, ssk, nw[0]);
               acc = fmaf(-d, d, acc);
             } else {
@@ -326,25 +244,19 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
           return s;
         };
 
-        // Inputs of butterfly utid + i*nthr; the next butterfly's are read
-        // before the current one's arithmetic (prev is read-only this step; in
-        // place, a thread's elements are its own).
+        // Inputs of butterfly tid + i*nthr; the next butterfly's are read
+        // before the current one's arithmetic (prev is read-only this step).
         auto read_in = [&](int i, float (&m)[R]) {
-          const int qq = min(utid + i * nthr, NB - 1);
-          if constexpr (kETab) {
+          const int qq = min(tid + i * nthr, NB - 1);
 #pragma unroll
-            for (int p = 0; p < R; ++p) m[p] = prev[ebase ^ Kel[p]];
-          } else {
-#pragma unroll
-            for (int p = 0; p < R; ++p) m[p] = prev[p * NB + qq];
-          }
+          for (int p = 0; p < R; ++p) m[p] = prev[p * NB + qq];
         };
         float nx[R];
         read_in(0, nx);
         float tmax = -INFINITY;
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
-          const int q = utid + i * nthr;
+          const int q = tid + i * nthr;
           float m[R];
 #pragma unroll
           for (int p = 0; p < R; ++p) m[p] = nx[p];
@@ -373,30 +285,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
               }
               store_vec<R>(cur + R * u, mo);
               tmax = max_with(tmax, mo);
-            } else if constexpr (kColUnroll) {
-              // Outputs unrolled, so every state's LUT offset is an immediate;
-              // a butterfly with an underflowed group is redone output by output.
-              float smin = 0.0f;
-#pragma unroll
-              for (int r = 0; r < R; ++r) {
-                float mo;
-                const float s = alpha_out(Fast{}, i, r, xu, u, m, oout, mo, (cbs[r] >> 2) + eoff);
-                smin = r ? fminf(smin, s) : s;
-                cur[ebase ^ Kel[r]] = mo;
-                tmax = vmax_raw(tmax, mo);
-              }
-              if constexpr (!EXACT) {
-                if (smin < kUnderflow) {
-#pragma unroll 1
-                  for (int r = 0; r < R; ++r) {
-                    float mo;
-                    alpha_out(std::true_type{}, i, r, xu, u, m, oout, mo,
-                              (hyb_col_base((uint32_t)(R * u + r), P.Q) >> 1) + eoff);
-                    cur[ebase ^ Kel[r]] = mo;
-                    tmax = vmax_raw(tmax, mo);
-                  }
-                }
-              }
             } else {
 #pragma unroll 1
               for (int r = 0; r < R; ++r) {
@@ -412,19 +300,11 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         }
         tmax = wave_max(tmax);
         if (lane == 0) wmax[(k & 1) * kMaxWaves + wave] = tmax;
-        rho = rho + KV >= nbits ? rho + KV - nbits : rho + KV;
         __syncthreads();
       }
 
-      // kETab: this thread's codewords, before the float4 table overwrites hcomp
-      float2 hv[kETab ? 4 : 1];
-      if constexpr (kETab) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) hv[j] = hcomp[tid + 256 * j];
-      }
-
       // log2 Z = C_{N-1} + LSE2 over the final reduced state.
-      const float* fin = mbuf + (kETab ? 0 : ((k + 1) & 1) * NT);
+      const float* fin = mbuf + ((k + 1) & 1) * NT;
       float Mz = -INFINITY;
       Mz = block_max(wmax + ((k + 1) & 1) * kMaxWaves);
       float part = 0.0f;
@@ -436,16 +316,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
       for (int w = 0; w < nwaves; ++w) Ssum += wsum[w];
       logZ2 = C + (double)Mz + (double)flog2(Ssum);
       // n~_{N-1} = 0: the buffer step N-1 of the beta sweep reads from.
-      for (int j = tid; j < NT; j += nthr) mbuf[(kETab ? 0 : ((k + 1) & 1) * NT) + j] = 0.0f;
-      if constexpr (kETab) {  // codewords of the float4 table (every wave read hcomp before the barrier above)
-        float4* et = reinterpret_cast<float4*>(lut);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int kk = tid + 256 * j;
-          et[kk] = make_float4(hv[j].x, hv[j].y, 0.0f, 0.0f);
-          et[kk + 1024] = make_float4(hv[j].x, hv[j].y, 0.0f, 0.0f);
-        }
-      }
+      for (int j = tid; j < NT; j += nthr) mbuf[((k + 1) & 1) * NT + j] = 0.0f;
       __syncthreads();
 
       // ------------------------------ beta sweep -------------------------------
@@ -453,7 +324,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
       // their use, across step boundaries (the next two in consumption order:
       // t descending, i ascending).
       auto slot_src = [&](int t, int i) {
-        const int q = min(utid + i * nthr, NB - 1);
+        const int q = min(tid + i * nthr, NB - 1);
         return slot + ((size_t)t * NB + q) * R;
       };
       float pa[R], pb[R];
@@ -462,17 +333,9 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         if (UPT > 1 || N > 1) load_vec<R>(UPT > 1 ? slot_src(N - 1, 1) : slot_src(N - 2, 0), pb);
       }
       double D = 0.0;  // D_t
-      // rho_t = kV * (t - 1) mod nb at t = N - 1 (kETab)
-      rho = (int)(((long long)KV * (N - 2) % nbits + nbits) % nbits);
       for (int t = N - 1; t >= 0; --t, ++k) {
-        const float* prev = mbuf + (kETab ? 0 : ((k + 1) & 1) * NT);
-        float* cur = mbuf + (kETab ? 0 : (k & 1) * NT);
-        const uint32_t ebase = kETab ? st_el((uint32_t)utid, rho) : 0u;
-        uint32_t Kel[kETab ? R : 1];
-        if constexpr (kETab) {
-#pragma unroll
-          for (int q = 0; q < R; ++q) Kel[q] = st_el((uint32_t)(q * NB), rho);
-        }
+        const float* prev = mbuf + ((k + 1) & 1) * NT;
+        float* cur = mbuf + (k & 1) * NT;
         float Qv = 0.0f;
         if (t != N - 1) {
           Qv = -INFINITY;
@@ -484,21 +347,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         float nw[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) nw[v] = -wbuf[t * V + v] * sk;
-        if constexpr (kETab) {  // every wave has left step t+1's table (barrier at its end)
-          float4* et = reinterpret_cast<float4*>(lut);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int kk = tid + 256 * j;
-            const float2 h = *reinterpret_cast<const float2*>(&et[kk]);
-            const float d0 = fmaf(h.x, ssk, nw[0]);
-            const float d1 = fmaf(h.y, ssk, nw[1]);
-            const float e = fmaf(-d1, d1, fmaf(-d0, d0, 0.0f));
-            et[kk].z = e;
-            et[kk + 1024].z = e;
-          }
-          __syncthreads();
-        }
-
         // Output p of butterfly u (unit i) from the shifted inputs nr[c]
         // (maximum 0): no = n~_{t-1}(p*NB + u) and the soft contribution
         // G * sum_c e_c h_c, with pms = raw m~_{t-1}(p*NB + u) + K_t - sh.
@@ -511,13 +359,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
           float y[R], hh[R][V];
 #pragma unroll
           for (int c = 0; c < R; ++c) {
-            if constexpr (kETab) {
-              const float4 he = *reinterpret_cast<const float4*>(lutb + cbs[c] + 2 * hyb_col_step(p, c));
-              y[c] = nr[c] + he.z;
-              hh[c][0] = he.x;
-              hh[c][1] = he.y;
-              continue;
-            }
             if (i < CU) {
 #pragma unroll
               for (int v = 0; v < V; ++v) hh[c][v] = hc[i < CU ? i : 0][p][c][v];
@@ -577,13 +418,8 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         };
 
         auto read_in = [&](int i, float (&n)[R]) {
-          const int qq = min(utid + i * nthr, NB - 1);
-          if constexpr (kETab) {
-#pragma unroll
-            for (int c = 0; c < R; ++c) n[c] = prev[ebase ^ Kel[c]];
-          } else {
-            load_vec<R>(prev + R * qq, n);
-          }
+          const int qq = min(tid + i * nthr, NB - 1);
+          load_vec<R>(prev + R * qq, n);
         };
         float nx[R];
         read_in(0, nx);
@@ -593,7 +429,7 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         float tmax = -INFINITY;
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
-          const int q = utid + i * nthr;
+          const int q = tid + i * nthr;
           float pm[R], n[R];
 #pragma unroll
           for (int r = 0; r < R; ++r) {
@@ -655,46 +491,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
                 cur[p * NB + u] = no[p];
               }
               tmax = max_with(tmax, no);
-            } else if constexpr (kColUnroll) {
-              // Outputs unrolled, so every state's LUT offset is an immediate;
-              // the butterfly's sums are redone when a group underflowed.
-              const float* src = slot_src(t, i);
-              float smin = 0.0f, ua[V], uh = 0.0f;
-#pragma unroll
-              for (int v = 0; v < V; ++v) ua[v] = 0.0f;
-#pragma unroll
-              for (int p = 0; p < R; ++p) {
-                float no, cs[V], hs;
-                const float pmr = src[p];
-                const float s = beta_out(Fast{}, i, p, xu, u, nr, n, pmr + kts, pmr, oout, no, cs, hs);
-                smin = p ? fminf(smin, s) : s;
-#pragma unroll
-                for (int v = 0; v < V; ++v) ua[v] += cs[v];
-                uh += hs;
-                cur[ebase ^ Kel[p]] = no;
-                tmax = vmax_raw(tmax, no);
-              }
-              if constexpr (!EXACT) {
-                if (smin < kUnderflow) {
-                  uh = 0.0f;
-#pragma unroll
-                  for (int v = 0; v < V; ++v) ua[v] = 0.0f;
-#pragma unroll 1
-                  for (int p = 0; p < R; ++p) {
-                    float no, cs[V], hs;
-                    const float pmr = src[p];
-                    beta_out(std::true_type{}, i, p, xu, u, nr, n, pmr + kts, pmr, oout, no, cs, hs);
-#pragma unroll
-                    for (int v = 0; v < V; ++v) ua[v] += cs[v];
-                    uh += hs;
-                    cur[ebase ^ Kel[p]] = no;
-                    tmax = vmax_raw(tmax, no);
-                  }
-                }
-              }
-              hacc += uh;
-#pragma unroll
-              for (int v = 0; v < V; ++v) acc[v] += ua[v];
             } else {
               const float* src = slot_src(t, i);
 #pragma unroll 1
@@ -725,7 +521,6 @@ __global__ __launch_bounds__(CODE == CODE_HYB_COL ? 256 : 512, CODE == CODE_HYB_
         }
         tmax = wave_max(tmax);
         if (lane == 0) wmax[(k & 1) * kMaxWaves + wave] = tmax;
-        rho = rho - KV < 0 ? rho - KV + nbits : rho - KV;
         __syncthreads();
       }
     };
@@ -767,13 +562,18 @@ const void* fwd_kernel_ptr(int KV, int V, int code, int upt, bool internals) {
   BCJR_FWD_UPTS(2, 1, CODE_3INST)
   BCJR_FWD_UPTS(2, 2, CODE_TABLE)
   BCJR_FWD_UPTS(2, 2, CODE_HYB)
-  // kV = 4: whole 16-state butterflies, at most 256 per sequence (L <= 16).
-  BCJR_FWD_CASE(4, 1, CODE_TABLE, 1)
-  BCJR_FWD_CASE(4, 1, CODE_1MAD, 1)
-  BCJR_FWD_CASE(4, 1, CODE_3INST, 1)
-  BCJR_FWD_CASE(4, 2, CODE_TABLE, 1)
-  BCJR_FWD_CASE(4, 2, CODE_HYB, 1)
-  BCJR_FWD_CASE(4, 2, CODE_HYB_COL, 1)
+  // kV = 4: the diagnostics forward, whole 16-state butterflies, at most 256 per
+  // sequence (L <= 16).
+  if (!internals) return nullptr;
+#define BCJR_FWD_DIAG16(V_, CODE_)    \
+  if (KV == 4 && V == V_ && code == CODE_ && upt == 1) \
+    return reinterpret_cast<const void*>(&bcjr_fwd_kernel<4, V_, CODE_, 1, 0, true>);
+  BCJR_FWD_DIAG16(1, CODE_TABLE)
+  BCJR_FWD_DIAG16(1, CODE_1MAD)
+  BCJR_FWD_DIAG16(1, CODE_3INST)
+  BCJR_FWD_DIAG16(2, CODE_TABLE)
+  BCJR_FWD_DIAG16(2, CODE_HYB)
+  BCJR_FWD_DIAG16(2, CODE_HYB_COL)
   return nullptr;
 }
 

@@ -52,6 +52,14 @@ const void* fwd_kernel_ptr(int KV, int V, int code, int upt, bool internals);
 // 1MAD / 3INST, 1024 threads, upt = 2^(L-14) butterflies per thread (L = 14..16).
 const void* fwd4_kernel_ptr(int code, int upt);
 const void* bwd_kernel_ptr(int KV, int V, int code, int upt);
+// The kV = 4 soft kernels (bcjr_soft16.h): kind 0 forward, 1 backward, 2 forward
+// with the marginal entropy; lpb lanes per butterfly.
+const void* soft16_kernel_ptr(int kind, int V, int code, int lpb);
+const void* soft16_col_kernel_ptr(int kind, int lpb);
+const void* soft16_hash_kernel_ptr(int kind, int code, int lpb);
+const void* soft16_hyb_kernel_ptr(int kind, int lpb);
+const void* soft16_table_kernel_ptr(int kind, int V, int lpb);
+hipError_t launch_transpose16(const float* table, float* out, int L, int V, hipStream_t stream);
 const void* vit_kernel_ptr(int KV, int V, int code, int upt, bool cache, bool wide);
 const void* decode_kernel_ptr(int KV, int V, int code);
 const void* trace_kernel_ptr(int KV, int V, int code);
@@ -93,12 +101,21 @@ inline size_t fwd4_lds_bytes(int L, int N) {
   return 8u * (size_t)((N + 1) & ~1) + 4u * (2 * NT + 3 * 16 + 4 + (size_t)N + 2 * 16);
 }
 
+// The layout at the head of bcjr_soft16_kernel.
+inline size_t soft16_lds_bytes(int L, int V, int N, int nwaves, int code, int Q, int kind) {
+  const size_t NT = (size_t)1 << (L - 4);
+  const size_t ns = (size_t)V + (kind ? 1 : 0);
+  const size_t apart = 2 * (size_t)nwaves * ns > 36 ? 2 * (size_t)nwaves * ns : 36;
+  const size_t tables = code == 4 ? 24576u : code == 3 ? (size_t)8 << Q : 0;
+  return tables + 4u * (kind == 1 ? 2 : 1) * NT + 8u * (size_t)((N + 1) & ~1) +
+         4u * (32 + apart + (size_t)N * V * (kind == 1 ? 2 : 1));
+}
+
 inline size_t bwd_lds_bytes(int L, int KV, int V, int N, int nwaves, int code, int Q) {
   const size_t NT = (size_t)1 << (L - KV);
   size_t b = 8u * (size_t)((N + 1) & ~1);
   b += 4u * (2 * NT + 4 * 16 + 2 * (size_t)N * V + 2 * (size_t)nwaves * (V + 1));
   if (code == 3) b += 8u + 8u * ((size_t)2 << Q);  // signed LUT, 8-byte aligned
-  if (code == 4) b += 8u + 32u * 64u * 8u;         // column-walk LUT (32 rows of 64)
   return b;
 }
 

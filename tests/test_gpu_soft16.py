@@ -1,0 +1,125 @@
+"""The kV = 4 soft kernels (csrc/bcjr_soft16.h) at the edges of their launch rules,
+against the float64 oracle: every L, odd and tiny N, batches on both sides of
+the two-halves rule, and workspaces that hold no transposed table or only part
+of the batch.  Tolerances are those of the other parity tests (float32
+log-domain recursions: soft 1e-4, gradient 1e-3, log Z 1e-5, entropy 1e-4)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SOFT_TOL, GRAD_TOL, Z_TOL = 1e-4, 1e-3, 1e-5
+
+
+def _codebook(bcjr, kind, L, V, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "hyb":
+        return bcjr.make_hyb_codebook_gpu(rng.standard_normal((512, 2)).astype(np.float32), 9, L, "cuda")
+    if kind == "3inst":
+        return bcjr.make_3inst_codebook(L, "cuda")
+    if kind == "1mad":
+        return bcjr.make_1mad_codebook(L, "cuda")
+    return torch.tensor(rng.standard_normal((1 << L, V)).astype(np.float32), device="cuda")
+
+
+def _rel(a, b):
+    return float(np.abs(a - b).max() / max(np.abs(b).max(), 1e-30))
+
+
+def _check(bcjr, oracle, kind, L, V, N, B, T, rows):
+    from bcjr import ops
+    k = 4 // V
+    cb = _codebook(bcjr, kind, L, V, L + N)
+    spec, table = bcjr.codes.resolve_codebook(cb, L, k, V, torch.device("cuda"))
+    rng = np.random.default_rng(100 * L + N)
+    x = rng.standard_normal((B, N, V)).astype(np.float32)
+    g = rng.standard_normal((B, N, V)).astype(np.float32)
+    gz = rng.standard_normal(B).astype(np.float32)
+    xd = torch.tensor(x, device="cuda")
+    soft, logZ = ops.forward(spec, xd, T, table)
+    soft_e, logZ_e, H = ops.forward_entropy(spec, xd, T, table)
+    d = ops.backward(spec, xd, T, table, torch.tensor(g, device="cuda"), torch.tensor(gz, device="cuda"))
+    cb_np, rows = cb.cpu().numpy(), [r for r in rows if r < B]
+    s_ref, z_ref = oracle.bcjr_forward(x[rows], cb_np, T, L, 4)
+    d_ref = oracle.bcjr_backward(x[rows], cb_np, T, L, 4, g[rows], gz[rows])
+    h_ref = oracle.marginal_entropy(x[rows], cb_np, T, L, 4)
+    assert _rel(soft.cpu().numpy()[rows], s_ref) < SOFT_TOL
+    assert _rel(logZ.cpu().numpy()[rows], z_ref) < Z_TOL
+    assert _rel(d.cpu().numpy()[rows], d_ref) < GRAD_TOL
+    assert np.abs(H.cpu().numpy()[rows] - h_ref).max() < 1e-4 * max(1.0, h_ref.max())
+    assert _rel(soft_e.cpu().numpy()[rows], s_ref) < SOFT_TOL and torch.isfinite(d).all()
+
+
+@pytest.mark.parametrize("kind,V", [("hyb", 2), ("table", 2), ("table", 1), ("3inst", 1), ("1mad", 1)])
+@pytest.mark.parametrize("L,N,T", [(8, 1, 0.3), (9, 2, 0.06), (10, 3, 0.3), (11, 37, 0.1), (12, 16, 0.06), (13, 5, 0.2),
+                                   (14, 4, 0.06), (15, 9, 0.1), (16, 1, 0.2), (16, 2, 0.05), (16, 7, 0.1)])
+def test_every_L_and_short_N(bcjr_mod, oracle, kind, V, L, N, T):
+    print(f"[soft16] {kind} V={V} L={L} N={N} T={T}", flush=True)
+    _check(bcjr_mod, oracle, kind, L, V, N, 3, T, [0, 1, 2])
+
+
+# 256 CUs: two halves on the wide column-walk workgroup up to 128, on the narrow
+# one up to half of what is resident, then one launch.
+@pytest.mark.parametrize("kind,V,L,B", [("hyb", 2, 16, 128), ("hyb", 2, 16, 129), ("hyb", 2, 16, 256), ("hyb", 2, 16, 257),
+                                        ("hyb", 2, 16, 600), ("table", 2, 16, 128), ("table", 2, 16, 129),
+                                        ("3inst", 1, 16, 300), ("hyb", 2, 12, 700), ("table", 1, 10, 2100)])
+@pytest.mark.parametrize("T", [0.06, 0.25])
+def test_batches_around_the_two_halves_rule(bcjr_mod, oracle, kind, V, L, B, T):
+    print(f"[soft16] {kind} L={L} B={B} T={T}", flush=True)
+    _check(bcjr_mod, oracle, kind, L, V, 6, B, T, [0, 127, 128, 255, 256, 299, 599, 2099])
+
+
+@pytest.mark.parametrize("kind,V", [("hyb", 2), ("table", 2)])
+def test_short_workspaces(bcjr_mod, oracle, kind, V):
+    """One slot only (no room for the meeting vectors or the table copy: whole
+    sequences, the table as it is), room for 3 of 8 sequences (three rounds of
+    halves, the same bits as one round), and the full workspace; a NaN sequence
+    and per-sequence T among them."""
+    from bcjr import _lib
+    lib = _lib.load()
+    L, N, B = 16, 12, 8
+    cb = _codebook(bcjr_mod, kind, L, V, 3)
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, 4 // V, V, torch.device("cuda"))
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((B, N, V)).astype(np.float32)
+    g = rng.standard_normal((B, N, V)).astype(np.float32)
+    T = np.array([0.05, 0.1, 0.2, 0.06, 0.5, 0.1, 0.3, 0.07], np.float32)
+    x[5, 3, 0] = np.nan
+    xd, gd, Td = (torch.tensor(a, device="cuda") for a in (x, g, T))
+    prob = spec.problem(B, N, True)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    nt = 1 << (L - 4)
+    outs = []
+    for op, st in ((0, 1), (1, 2)):
+        full = ctypes.c_size_t(0)
+        _lib.check(lib.bcjr_workspace_bytes(ctypes.byref(prob), op, ctypes.byref(full)), "ws")
+        slot = N * nt * 4 * st
+        per = slot + 2 * nt * 4 * st + 256
+        copy = 4 * V << L if kind == "table" else 0
+        res = []
+        for nbytes in (full.value, copy + 3 * per, slot):
+            print(f"[soft16] {kind} op {op} workspace {nbytes}", flush=True)
+            ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device="cuda")
+            out, z = torch.full((B, N, V), 7.0, device="cuda"), torch.full((B,), 7.0, device="cuda")
+            if op == 0:
+                rc = lib.bcjr_forward(ctypes.byref(prob), xd.data_ptr(), Td.data_ptr(), _lib.ptr(table), out.data_ptr(),
+                                      z.data_ptr(), ws.data_ptr(), nbytes, stream)
+            else:
+                rc = lib.bcjr_backward(ctypes.byref(prob), xd.data_ptr(), Td.data_ptr(), _lib.ptr(table), None,
+                                       gd.data_ptr(), None, out.data_ptr(), ws.data_ptr(), nbytes, stream)
+            _lib.check(rc, "call")
+            torch.cuda.synchronize()
+            assert torch.isnan(out[5]).all()
+            res.append(out.cpu().numpy())
+        assert np.array_equal(res[0], res[1], equal_nan=True)
+        outs.append(res)
+    rows = [0, 1, 2, 3, 4, 6, 7]
+    cb_np = cb.cpu().numpy()
+    for r in rows:
+        s_ref, _ = oracle.bcjr_forward(x[r:r + 1], cb_np, float(T[r]), L, 4)
+        d_ref = oracle.bcjr_backward(x[r:r + 1], cb_np, float(T[r]), L, 4, g[r:r + 1])
+        for i in (0, 2):
+            assert _rel(outs[0][i][r], s_ref[0]) < SOFT_TOL and _rel(outs[1][i][r], d_ref[0]) < GRAD_TOL
