@@ -33,9 +33,19 @@
 // the LUT's entries (below).  CODE_TABLE reads c(s) at p SP + c SC + u SU floats
 // times V: with the transposed copy the host makes in the workspace (SC = NB, SU = 1)
 // a wave's lanes, which hold consecutive u, read consecutive addresses; in the
-// natural order (SC = 1, SU = 16) each lane reads a cache line of its own, and the
-// forward ran TABLENAT.  The other codes hash each state, HYB
-// through the LUT in LDS.
+// natural order (SC = 1, SU = 16) each lane reads a cache line of its own (500
+// sequences of 128 steps at L = 16, V = 2: forward 4.87 against 23.2 ms, backward
+// 5.06 against 17.3 ms).  The other codes hash each state, HYB through the LUT in
+// LDS.
+//
+// Bounds.  Large batches: VALU issue (column walk, L = 16, T = 0.1: 9.6 VALU
+// instructions per cell forward and 17.2 backward in the step bodies, plus about
+// 190 per wave and step), then the tables' barrier; small ones: the latency of a
+// step, N/2 of them each way.  Measured against one 256-thread workgroup per
+// sequence with a butterfly per lane, at N = 128, HYB Q = 9: 8 sequences forward
+// 1.61 -> 0.62 ms, backward 2.67 -> 0.85 ms; 4,096 sequences 15.4 -> 13.5-14.3 ms
+// and 24.5 -> 23.6 ms; L = 12, 128 sequences (16 butterflies) 2.71 -> 0.21 ms and
+// 3.62 -> 0.24 ms; a table at L = 16, 500 sequences 24.7 -> 4.9 and 24.0 -> 5.1 ms.
 #pragma once
 
 #include "bcjr_device.h"
