@@ -321,9 +321,35 @@ int make_soft16_plan(const bcjr_problem* p, int op, bool wide, const DeviceInfo&
   return finish_plan(p, di, pl);
 }
 
+// The two-halves soft kernels of kV <= 2 (bcjr_halves.h), up to 1,024 threads:
+// kV = 2 whole butterflies from L = 12 on, else a lane per output (N = 256, forward
+// and backward, whole butterflies against a lane per output: L = 13, 128 sequences
+// 0.28 against 0.37 and 0.41 against 0.49 ms; L = 12 0.24 against 0.27 and 0.32
+// against 0.32 ms; L = 10, 64 sequences 0.21 against 0.18 and 0.26 against 0.21 ms).
+int make_halves_plan(const bcjr_problem* p, int op, const DeviceInfo& di, Plan* pl) {
+  const int KV = p->k * p->V, kind = op == OP_BWD ? 1 : op == OP_FWD_ENTROPY ? 2 : 0;
+  const int lpb = KV == 2 && p->L >= 12 ? 1 : 1 << KV;
+  pl->KV = KV;
+  pl->R = 1 << KV;
+  pl->NSUB = 1;
+  pl->NT = 1 << (p->L - KV);
+  pl->NB = pl->NT >> KV;
+  pl->NU = pl->NB;
+  pl->upt = std::max(1, pl->NB * lpb / 1024);
+  pl->nthr = std::max(64, pl->NB * lpb / pl->upt);
+  pl->fn = bcjr::halves_kernel_ptr(kind, KV, p->V, p->code, pl->upt, lpb);
+  if (!pl->fn) return fail(BCJR_EUNSUPPORTED, "no two-halves kernel for L=%d k=%d V=%d code=%d", p->L, p->k, p->V, p->code);
+  pl->lds = bcjr::halves_lds_bytes(p->L, KV, p->V, (int)p->N, pl->nthr / 64, p->code, p->Q, kind,
+                                   bcjr::halves_in_place(op == OP_BWD, pl->upt, lpb));
+  pl->swz = pick_swizzle(p->L, KV);
+  pl->slot_bytes = slot_bytes_of(p, op == OP_BWD ? OP_BWD : OP_FWD);
+  return finish_plan(p, di, pl);
+}
+
 int make_plan_uncached(const bcjr_problem* p, int op, bool wide, const DeviceInfo& di, Plan* pl) {
   const int KV = p->k * p->V, R = 1 << KV, RO = R < 4 ? R : 4;
   if (KV == 4 && (op == OP_FWD || op == OP_BWD || op == OP_FWD_ENTROPY)) return make_soft16_plan(p, op, wide, di, pl);
+  if (wide && op != OP_VIT) return make_halves_plan(p, op, di, pl);
   if (op == OP_FWD_ENTROPY) op = OP_FWD_INTERNALS;
   pl->KV = KV;
   pl->R = R;
@@ -428,18 +454,32 @@ size_t halves_bytes(const bcjr_problem* p, int op) {
          round256(((size_t)p->N + 2) * sizeof(double));
 }
 
-// Whether a kV = 4 soft call runs its sequences in two halves each (bcjr_soft16.h),
-// on which plan: when twice as many workgroups still all fit at once, so that
-// the steps in sequence are halved and no sequence waits for another.  The choice
-// depends on the problem and the device only, not on the workspace (a short one
-// takes several rounds), so every workspace gives the same bits.  Column walk:
-// one workgroup of twice the threads per CU where that is all there is.
-// MEASURED16
+// Whether a soft call runs its sequences in two halves each (bcjr_soft16.h,
+// bcjr_halves.h), and on which plan: when twice as many workgroups still all fit
+// at once, so that the steps in sequence are halved and no sequence waits for
+// another.  The choice depends on the problem and the device only, not on the
+// workspace (a short one takes several rounds), so every workspace gives the same
+// bits.  kV = 4: the plan of one launch, or, column walk, one workgroup of twice
+// the threads per CU where that is all there is.
+// Measured, forward and backward, one launch -> two halves, N = 128: column walk
+// 8 sequences 1.17 -> 0.62 and 1.83 -> 0.85 ms (narrow workgroup 0.70 and 1.01),
+// 128 sequences 1.27 -> 0.70 and 1.95 -> 0.98 ms (0.79 and 1.11), 256 sequences on
+// the narrow one 1.28 -> 1.07 and 1.97 -> 1.61 ms; a table, 128 sequences 2.44 ->
+// 1.15 and 2.51 -> 1.43 ms; L = 12, 256 sequences 0.38 -> 0.26 and 0.42 -> 0.29 ms.
 int halves_plan(const bcjr_problem* p, int op, const Plan& pl, Plan* out, bool* halves) {
-  *halves = p->N >= 2 && 2 * p->B <= pl.max_blocks;
-  *out = pl;
-  if (*halves && bcjr::soft_kernel_code(p->code, p->L, 4, p->Q) == bcjr::CODE_HYB_COL && 2 * p->B <= pl.num_cu)
-    return make_plan(p, op, out, true);
+  *halves = false;
+  if (p->N < 2) return BCJR_OK;
+  if (pl.KV == 4) {
+    *halves = 2 * p->B <= pl.max_blocks;
+    *out = pl;
+    if (*halves && bcjr::soft_kernel_code(p->code, p->L, 4, p->Q) == bcjr::CODE_HYB_COL && 2 * p->B <= pl.num_cu)
+      return make_plan(p, op, out, true);
+    return BCJR_OK;
+  }
+  const int rc = make_plan(p, op, out, true);
+  if (rc == BCJR_EUNSUPPORTED) return BCJR_OK;  // its LDS does not hold this N (or Q): one launch
+  if (rc) return rc;
+  *halves = 2 * p->B <= out->max_blocks;
   return BCJR_OK;
 }
 
@@ -448,17 +488,55 @@ size_t table16_bytes(const bcjr_problem* p) {
   return p->k * p->V == 4 && p->code == BCJR_CODE_TABLE ? round256(((size_t)p->V << p->L) * sizeof(float)) : 0;
 }
 
-// One kV = 4 soft call: the table's transposed copy (when the workspace has room
-// for it beside one slot; else the kernels read the table as it is), then the
-// batch in two halves or in one launch.
-int launch_soft16(const bcjr_problem* p, int op, bcjr::Soft16Params P, void* ws, size_t ws_bytes,
-                  hipStream_t stream) {
+// The two launches of a batch in two halves, over as many sequences a round as the
+// workspace holds; *done = false when it does not hold one.
+int launch_halves(const bcjr_problem* p, int op, const Plan& pl, bcjr::Soft16Params P, char* ws, size_t ws_bytes,
+                  hipStream_t stream, bool* done) {
+  const long long round = std::min<long long>(p->B, (long long)(ws_bytes / halves_bytes(p, op)));
+  *done = round >= 1;
+  if (!*done) return BCJR_OK;
+  const size_t st = op == OP_BWD ? 2 : 1, row = (size_t)p->N * p->V;
+  char* mid = ws + (size_t)round * pl.slot_bytes;
+  P.ws = reinterpret_cast<float*>(ws);
+  P.mid = reinterpret_cast<float*>(mid);
+  P.moff = reinterpret_cast<double*>(mid + (size_t)round * round256(2 * st * pl.NT * sizeof(float)));
+  P.swz = pl.swz;
+  for (long long b0 = 0; b0 < p->B; b0 += round) {
+    bcjr::Soft16Params H = P;
+    H.B = std::min<long long>(round, p->B - b0);
+    H.seq += b0 * row;
+    H.out += b0 * row;
+    if (P.t_per_seq) H.T += b0;
+    if (H.logZ) H.logZ += b0;
+    if (H.H_out) H.H_out += b0 * p->N;
+    if (H.g_soft) H.g_soft += b0 * row;
+    if (H.g_logZ) H.g_logZ += b0;
+    for (int mode : {(int)bcjr::SOFT_FIRST, (int)bcjr::SOFT_SECOND}) {
+      H.mode = mode;
+      void* args[] = {&H};
+      hipError_t e = hipLaunchKernel(pl.fn, dim3((unsigned)(2 * H.B)), dim3((unsigned)pl.nthr), args, pl.lds, stream);
+      if (e != hipSuccess) return hip_fail(e, "hipLaunchKernel");
+      e = hipGetLastError();
+      if (e != hipSuccess) return hip_fail(e, "kernel launch");
+    }
+  }
+  return BCJR_OK;
+}
+
+// One soft call on the kV = 4 kernels, or in two halves: the table's transposed
+// copy (kV = 4, when the workspace has room for it beside one slot; else the
+// kernels read the table as it is), then the batch in two halves or in one launch.
+// *done = false: the call is one for the whole-sequence kernels of kV <= 2.
+int launch_soft(const bcjr_problem* p, int op, bcjr::Soft16Params P, void* ws, size_t ws_bytes, hipStream_t stream,
+                bool* done) {
   Plan pl, hp;
+  *done = false;
   int rc = make_plan(p, op, &pl);
   if (rc) return rc;
   bool halves = false;
   rc = halves_plan(p, op, pl, &hp, &halves);
   if (rc) return rc;
+  if (pl.KV != 4 && !halves) return BCJR_OK;
   char* w = static_cast<char*>(ws);
   size_t left = ws_bytes;
   P.SC = 1;
@@ -477,39 +555,18 @@ int launch_soft16(const bcjr_problem* p, int op, bcjr::Soft16Params P, void* ws,
   P.L = p->L;
   P.Q = p->Q;
   P.t_per_seq = p->t_per_seq ? 1 : 0;
+  P.slot_floats = pl.slot_bytes / sizeof(float);
+  if (halves) {
+    rc = launch_halves(p, op, hp, P, w, left, stream, done);
+    if (rc || *done) return rc;
+  }
+  if (pl.KV != 4) return BCJR_OK;
+  *done = true;
   P.swz = pl.swz;
   P.ws = reinterpret_cast<float*>(w);
-  P.slot_floats = pl.slot_bytes / sizeof(float);
-  const size_t per = halves_bytes(p, op);
-  const long long round = halves ? std::min<long long>(p->B, (long long)(left / per)) : 0;
-  if (round < 1) {
-    P.mode = 0;
-    P.B = p->B;
-    return launch(pl, p->B, left, &P, stream);
-  }
-  const size_t NT = (size_t)pl.NT, st = op == OP_BWD ? 2 : 1, row = (size_t)p->N * p->V;
-  char* mid = w + (size_t)round * pl.slot_bytes;
-  P.mid = reinterpret_cast<float*>(mid);
-  P.moff = reinterpret_cast<double*>(mid + (size_t)round * round256(2 * st * NT * sizeof(float)));
-  for (long long b0 = 0; b0 < p->B; b0 += round) {
-    bcjr::Soft16Params H = P;
-    H.B = std::min<long long>(round, p->B - b0);
-    H.seq += b0 * row;
-    H.out += b0 * row;
-    if (P.t_per_seq) H.T += b0;
-    if (H.logZ) H.logZ += b0;
-    if (H.H_out) H.H_out += b0 * p->N;
-    if (H.g_soft) H.g_soft += b0 * row;
-    if (H.g_logZ) H.g_logZ += b0;
-    for (H.mode = 1; H.mode <= 2; ++H.mode) {
-      void* args[] = {&H};
-      hipError_t e = hipLaunchKernel(hp.fn, dim3((unsigned)(2 * H.B)), dim3((unsigned)hp.nthr), args, hp.lds, stream);
-      if (e != hipSuccess) return hip_fail(e, "hipLaunchKernel");
-      e = hipGetLastError();
-      if (e != hipSuccess) return hip_fail(e, "kernel launch");
-    }
-  }
-  return BCJR_OK;
+  P.mode = bcjr::SOFT_WHOLE;
+  P.B = p->B;
+  return launch(pl, p->B, left, &P, stream);
 }
 
 // Sequence slots of bcjr_forward_noalloc: a static device array, one copy per
@@ -590,7 +647,7 @@ int bcjr_workspace_bytes(const bcjr_problem* prob, int op, size_t* bytes) {
   if (rc) return rc;
   const long long slots = std::max<long long>(1, std::min<long long>(prob->B, pl.max_blocks));
   *bytes = (size_t)slots * pl.slot_bytes;
-  if (pl.KV == 4 && op != OP_VIT) {
+  if (op != OP_VIT) {
     Plan hp;
     bool halves = false;
     rc = halves_plan(prob, op, pl, &hp, &halves);
@@ -608,17 +665,17 @@ int bcjr_forward(const bcjr_problem* prob, const float* seq, const float* T, con
   if (!seq || !T || !soft || !ws) return fail(BCJR_EINVAL, "seq, T, soft and ws must be non-NULL");
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
-  if (prob->k * prob->V == 4) {
-    bcjr::Soft16Params S = {};
-    S.seq = seq;
-    S.T = T;
-    S.table = codebook_or_lut;
-    S.out = soft;
-    S.logZ = logZ;
-    return launch_soft16(prob, OP_FWD, S, ws, ws_bytes, stream);
-  }
+  bcjr::Soft16Params S = {};
+  S.seq = seq;
+  S.T = T;
+  S.table = codebook_or_lut;
+  S.out = soft;
+  S.logZ = logZ;
+  bool done = false;
+  int rc = launch_soft(prob, OP_FWD, S, ws, ws_bytes, stream, &done);
+  if (rc || done) return rc;
   Plan pl;
-  int rc = make_plan(prob, OP_FWD, &pl);
+  rc = make_plan(prob, OP_FWD, &pl);
   if (rc) return rc;
   bcjr::FwdParams P = {};
   P.seq = seq;
@@ -677,7 +734,18 @@ int bcjr_forward_internals(const bcjr_problem* prob, const float* seq, const flo
   P.L = prob->L;
   P.Q = prob->Q;
   P.t_per_seq = prob->t_per_seq ? 1 : 0;
-  return launch(pl, prob->B, ws_bytes, &P, stream);
+  rc = launch(pl, prob->B, ws_bytes, &P, stream);
+  if (rc) return rc;
+  // soft and log Z as bcjr_forward gives them, bit for bit, where it runs other
+  // kernels than the diagnostics one (whose own values these overwrite).
+  bcjr::Soft16Params S = {};
+  S.seq = seq;
+  S.T = T;
+  S.table = codebook_or_lut;
+  S.out = soft;
+  S.logZ = logZ;
+  bool done = false;
+  return launch_soft(prob, OP_FWD, S, ws, ws_bytes, stream, &done);
 }
 
 int bcjr_forward_entropy(const bcjr_problem* prob, const float* seq, const float* T,
@@ -689,18 +757,18 @@ int bcjr_forward_entropy(const bcjr_problem* prob, const float* seq, const float
     return fail(BCJR_EINVAL, "seq, T, soft, ws and entropy must be non-NULL");
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
-  if (prob->k * prob->V == 4) {
-    bcjr::Soft16Params S = {};
-    S.seq = seq;
-    S.T = T;
-    S.table = codebook_or_lut;
-    S.out = soft;
-    S.logZ = logZ;
-    S.H_out = entropy;
-    return launch_soft16(prob, OP_FWD_ENTROPY, S, ws, ws_bytes, stream);
-  }
+  bcjr::Soft16Params S = {};
+  S.seq = seq;
+  S.T = T;
+  S.table = codebook_or_lut;
+  S.out = soft;
+  S.logZ = logZ;
+  S.H_out = entropy;
+  bool done = false;
+  int rc = launch_soft(prob, OP_FWD_ENTROPY, S, ws, ws_bytes, stream, &done);
+  if (rc || done) return rc;
   Plan pl;
-  int rc = make_plan(prob, OP_FWD_ENTROPY, &pl);
+  rc = make_plan(prob, OP_FWD_ENTROPY, &pl);
   if (rc) return rc;
   bcjr::FwdParams P = {};
   P.seq = seq;
@@ -728,18 +796,18 @@ int bcjr_backward(const bcjr_problem* prob, const float* seq, const float* T, co
     return fail(BCJR_EINVAL, "seq, T, g_soft, g_seq and ws must be non-NULL");
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
-  if (prob->k * prob->V == 4) {
-    bcjr::Soft16Params S = {};
-    S.seq = seq;
-    S.T = T;
-    S.table = codebook_or_lut;
-    S.out = g_seq;
-    S.g_soft = g_soft;
-    S.g_logZ = g_logZ;
-    return launch_soft16(prob, OP_BWD, S, ws, ws_bytes, stream);
-  }
+  bcjr::Soft16Params S = {};
+  S.seq = seq;
+  S.T = T;
+  S.table = codebook_or_lut;
+  S.out = g_seq;
+  S.g_soft = g_soft;
+  S.g_logZ = g_logZ;
+  bool done = false;
+  int rc = launch_soft(prob, OP_BWD, S, ws, ws_bytes, stream, &done);
+  if (rc || done) return rc;
   Plan pl;
-  int rc = make_plan(prob, OP_BWD, &pl);
+  rc = make_plan(prob, OP_BWD, &pl);
   if (rc) return rc;
   bcjr::BwdParams P = {};
   P.seq = seq;

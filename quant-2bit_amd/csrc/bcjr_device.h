@@ -539,7 +539,12 @@ struct BwdParams {
   Swizzle swz;          // LDS layout of (m~, mu) and (n~, nu)
 };
 
-// The kV = 4 soft kernels (bcjr_soft16.h).
+// Launch modes (Soft16Params::mode): whole sequences, or the first or second
+// launch of the two-halves scheme.
+enum { SOFT_WHOLE = 0, SOFT_FIRST = 1, SOFT_SECOND = 2 };
+
+// The kV = 4 soft kernels (bcjr_soft16.h) and the two-halves kernels of kV <= 2
+// (bcjr_halves.h).
 struct Soft16Params {
   const float* seq;      // (B, N, V)
   const float* T;        // (B,) or (1,)

@@ -59,6 +59,11 @@ const void* soft16_col_kernel_ptr(int kind, int lpb);
 const void* soft16_hash_kernel_ptr(int kind, int code, int lpb);
 const void* soft16_hyb_kernel_ptr(int kind, int lpb);
 const void* soft16_table_kernel_ptr(int kind, int V, int lpb);
+// The two-halves soft kernels of kV <= 2 (bcjr_halves.h): upt butterflies per
+// thread with lpb = 1 lane each, or upt = 1 with lpb = 2^kV; null when not built.
+const void* halves_kernel_ptr(int kind, int KV, int V, int code, int upt, int lpb);
+const void* halves_bwd_kernel_ptr(int KV, int V, int code, int upt, int lpb);
+const void* halves_entropy_kernel_ptr(int KV, int V, int code, int upt, int lpb);
 hipError_t launch_transpose16(const float* table, float* out, int L, int V, hipStream_t stream);
 const void* vit_kernel_ptr(int KV, int V, int code, int upt, bool cache, bool wide);
 const void* decode_kernel_ptr(int KV, int V, int code);
@@ -99,6 +104,19 @@ inline size_t fwd_lds_bytes(int L, int KV, int V, int N, int nwaves, int code, i
 inline size_t fwd4_lds_bytes(int L, int N) {
   const size_t NT = (size_t)1 << (L - 2);
   return 8u * (size_t)((N + 1) & ~1) + 4u * (2 * NT + 3 * 16 + 4 + (size_t)N + 2 * 16);
+}
+
+// The state of a two-halves kernel is updated in place, not double-buffered.
+__host__ __device__ constexpr bool halves_in_place(bool grad, int upt, int lpb) { return grad && upt == 4 && lpb == 1; }
+
+// The layout at the head of bcjr_halves_kernel.
+inline size_t halves_lds_bytes(int L, int KV, int V, int N, int nwaves, int code, int Q, int kind,
+                               bool in_place) {
+  const size_t NT = (size_t)1 << (L - KV);
+  const size_t ns = (size_t)V + (kind ? 1 : 0);
+  const size_t apart = 2 * (size_t)nwaves * ns > 36 ? 2 * (size_t)nwaves * ns : 36;
+  return (code == 3 ? (size_t)16 << Q : 0) + 4u * (kind == 1 ? 2 : 1) * (in_place ? 1 : 2) * NT + 8u * (size_t)((N + 1) & ~1) +
+         4u * (32 + apart + (size_t)N * V * (kind == 1 ? 2 : 1));
 }
 
 // The layout at the head of bcjr_soft16_kernel.

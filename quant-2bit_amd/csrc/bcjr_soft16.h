@@ -53,9 +53,6 @@
 
 namespace bcjr {
 
-// Launch modes (Soft16Params::mode).
-enum { SOFT16_WHOLE = 0, SOFT16_FIRST = 1, SOFT16_SECOND = 2 };
-
 // Threads of a workgroup and waves per SIMD the instance is built for.
 template <int CODE, int LPB, bool GRAD>
 struct Soft16Shape {
@@ -123,9 +120,9 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
     return (kCol && !GRAD ? col_walk_state_el(y) : swizzle(y, swz)) << LGB;
   };
 
-  for (long long b = P.mode == SOFT16_WHOLE ? blockIdx.x : blockIdx.x >> 1; b < P.B;
-       b += P.mode == SOFT16_WHOLE ? gridDim.x : (P.B + 1)) {
-    const size_t slot_id = P.mode == SOFT16_WHOLE ? (size_t)blockIdx.x : (size_t)b;
+  for (long long b = P.mode == SOFT_WHOLE ? blockIdx.x : blockIdx.x >> 1; b < P.B;
+       b += P.mode == SOFT_WHOLE ? gridDim.x : (P.B + 1)) {
+    const size_t slot_id = P.mode == SOFT_WHOLE ? (size_t)blockIdx.x : (size_t)b;
     float* slot = P.ws + slot_id * P.slot_floats;
     const float Tb = P.T[P.t_per_seq ? b : 0];
     const float sk = sqrtf(kLog2e / Tb);
@@ -134,7 +131,7 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
     const float twoT = 2.0f / Tb;
     const float* seqb = P.seq + (size_t)b * N * V;
     float* outb = P.out + (size_t)b * N * V;
-    const int role = P.mode == SOFT16_WHOLE ? 0 : (int)(blockIdx.x & 1);  // two halves: 0 alpha, 1 beta
+    const int role = P.mode == SOFT_WHOLE ? 0 : (int)(blockIdx.x & 1);  // two halves: 0 alpha, 1 beta
 
     // T must be finite and > 0, the weights and upstream gradients finite;
     // otherwise the sequence's outputs are NaN.
@@ -154,7 +151,7 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
     if (bad) *bflag = 1;
     __syncthreads();
     if (*bflag) {  // uniform: every thread reads the flag after the barrier
-      if (role == 0 && P.mode != SOFT16_FIRST) {
+      if (role == 0 && P.mode != SOFT_FIRST) {
         for (int i = tid; i < N * V; i += nthr) outb[i] = NAN;
         if (tid == 0 && !GRAD && P.logZ) P.logZ[b] = NAN;
         if constexpr (ENT)
@@ -756,7 +753,7 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
     auto run = [&](auto exact) __attribute__((always_inline)) {
       using F = std::false_type;
       using Y = std::true_type;
-      if (P.mode == SOFT16_WHOLE) {
+      if (P.mode == SOFT_WHOLE) {
         fill_state((float)KV);  // m~_{-1} = log2(R)
         __syncthreads();
         const double C = sweep(F{}, F{}, exact, 0, N, 0.0, (float)KV);
@@ -769,7 +766,7 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
       const int h = N / 2;
       float* mid = P.mid + (size_t)b * 2 * ST * NT;
       double* moff = P.moff + (size_t)b * (N + 2);
-      if (P.mode == SOFT16_FIRST) {
+      if (P.mode == SOFT_FIRST) {
         fill_state(role ? 0.0f : (float)KV);
         __syncthreads();
         double off;
@@ -795,7 +792,7 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
     } else {
       run(std::false_type{});
     }
-    if (!GRAD && P.mode != SOFT16_FIRST && role == 0 && tid == 0 && P.logZ) P.logZ[b] = (float)(logZ2 * kLn2);
+    if (!GRAD && P.mode != SOFT_FIRST && role == 0 && tid == 0 && P.logZ) P.logZ[b] = (float)(logZ2 * kLn2);
     __syncthreads();
   }
 }

@@ -123,3 +123,55 @@ def test_short_workspaces(bcjr_mod, oracle, kind, V):
         d_ref = oracle.bcjr_backward(x[r:r + 1], cb_np, float(T[r]), L, 4, g[r:r + 1])
         for i in (0, 2):
             assert _rel(outs[0][i][r], s_ref[0]) < SOFT_TOL and _rel(outs[1][i][r], d_ref[0]) < GRAD_TOL
+
+
+@pytest.mark.parametrize("kind,k,V,L,N", [("table", 1, 1, 2, 5), ("table", 1, 1, 7, 64), ("table", 1, 1, 11, 33),
+                                          ("3inst", 2, 1, 4, 2), ("1mad", 2, 1, 6, 3), ("table", 2, 1, 9, 17),
+                                          ("3inst", 2, 1, 12, 40), ("1mad", 2, 1, 13, 21), ("3inst", 2, 1, 14, 8),
+                                          ("table", 2, 1, 15, 9), ("3inst", 2, 1, 16, 11), ("1mad", 2, 1, 16, 1),
+                                          ("hyb", 1, 2, 8, 7), ("table", 1, 2, 12, 30), ("hyb", 1, 2, 13, 5),
+                                          ("table", 1, 2, 15, 4), ("hyb", 1, 2, 16, 6)])
+@pytest.mark.parametrize("T", [0.06, 0.2])
+def test_small_steps_in_two_halves(bcjr_mod, oracle, kind, k, V, L, N, T):
+    """kV <= 2 (csrc/bcjr_halves.h): every L's launch shape, odd and even N, a
+    table, hashed codes and the LUT."""
+    from bcjr import ops
+    print(f"[halves] {kind} k={k} V={V} L={L} N={N} T={T}", flush=True)
+    cb = _codebook(bcjr_mod, kind, L, V, L + N)
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, k, V, torch.device("cuda"))
+    rng, B = np.random.default_rng(L * 7 + N), 3
+    x = rng.standard_normal((B, N, V)).astype(np.float32)
+    g = rng.standard_normal((B, N, V)).astype(np.float32)
+    gz = rng.standard_normal(B).astype(np.float32)
+    Tv = np.array([T, 0.5, 0.1], np.float32)
+    xd, Td = torch.tensor(x, device="cuda"), torch.tensor(Tv, device="cuda")
+    soft, logZ = ops.forward(spec, xd, Td, table)
+    _, _, H = ops.forward_entropy(spec, xd, Td, table)
+    d = ops.backward(spec, xd, Td, table, torch.tensor(g, device="cuda"), torch.tensor(gz, device="cuda"))
+    cb_np = cb.cpu().numpy()
+    for r in range(B):
+        s_ref, z_ref = oracle.bcjr_forward(x[r:r + 1], cb_np, float(Tv[r]), L, k * V)
+        d_ref = oracle.bcjr_backward(x[r:r + 1], cb_np, float(Tv[r]), L, k * V, g[r:r + 1], gz[r:r + 1])
+        h_ref = oracle.marginal_entropy(x[r:r + 1], cb_np, float(Tv[r]), L, k * V)
+        assert _rel(soft.cpu().numpy()[r], s_ref[0]) < SOFT_TOL and _rel(logZ.cpu().numpy()[r], z_ref[0]) < Z_TOL
+        assert _rel(d.cpu().numpy()[r], d_ref[0]) < GRAD_TOL
+        assert np.abs(H.cpu().numpy()[r] - h_ref[0]).max() < 1e-4 * max(1.0, h_ref.max())
+
+
+@pytest.mark.parametrize("B", [128, 129])
+def test_sequences_beside_each_other_in_two_halves(bcjr_mod, oracle, B):
+    """The largest batch two halves take at L = 16 (one workgroup per CU) and the
+    smallest one launch takes: first, middle and last sequence."""
+    from bcjr import ops
+    print(f"[halves] 3inst L=16 B={B}", flush=True)
+    L, N, T = 16, 10, 0.1
+    cb = bcjr_mod.make_3inst_codebook(L, "cuda")
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, 2, 1, torch.device("cuda"))
+    rng = np.random.default_rng(B)
+    x, g = (rng.standard_normal((B, N, 1)).astype(np.float32) for _ in range(2))
+    xd = torch.tensor(x, device="cuda")
+    soft, _ = ops.forward(spec, xd, T, table)
+    d = ops.backward(spec, xd, T, table, torch.tensor(g, device="cuda"))
+    rows = [0, 64, B - 1]
+    assert _rel(soft.cpu().numpy()[rows], oracle.bcjr_forward(x[rows], cb.cpu().numpy(), T, L, 2)[0]) < SOFT_TOL
+    assert _rel(d.cpu().numpy()[rows], oracle.bcjr_backward(x[rows], cb.cpu().numpy(), T, L, 2, g[rows])) < GRAD_TOL
