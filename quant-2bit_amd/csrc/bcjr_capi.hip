@@ -488,6 +488,29 @@ size_t table16_bytes(const bcjr_problem* p) {
   return p->k * p->V == 4 && p->code == BCJR_CODE_TABLE ? round256(((size_t)p->V << p->L) * sizeof(float)) : 0;
 }
 
+// A Viterbi launch; kV = 4 tables first get their transposed copy, as above.
+int launch_viterbi(const bcjr_problem* p, bcjr::VitParams P, void* ws, size_t ws_bytes, hipStream_t stream) {
+  Plan pl;
+  const int rc = make_plan(p, OP_VIT, &pl);
+  if (rc) return rc;
+  char* w = static_cast<char*>(ws);
+  const size_t tb = table16_bytes(p);
+  P.tab16 = P.table;
+  P.SC = 1;
+  P.SU = 16;
+  if (tb && ws_bytes >= tb + pl.slot_bytes) {
+    hipError_t e = bcjr::launch_transpose16(P.table, reinterpret_cast<float*>(w), p->L, p->V, stream);
+    if (e != hipSuccess) return hip_fail(e, "codebook transpose launch");
+    P.tab16 = reinterpret_cast<const float*>(w);
+    P.SC = (uint32_t)pl.NB;
+    P.SU = 1;
+    w += tb;
+    ws_bytes -= tb;
+  }
+  P.ws = reinterpret_cast<uint8_t*>(w);
+  return launch(pl, p->B, ws_bytes, &P, stream);
+}
+
 // The two launches of a batch in two halves, over as many sequences a round as the
 // workspace holds; *done = false when it does not hold one.
 int launch_halves(const bcjr_problem* p, int op, const Plan& pl, bcjr::Soft16Params P, char* ws, size_t ws_bytes,
@@ -653,8 +676,8 @@ int bcjr_workspace_bytes(const bcjr_problem* prob, int op, size_t* bytes) {
     rc = halves_plan(prob, op, pl, &hp, &halves);
     if (rc) return rc;
     if (halves) *bytes = std::max(*bytes, (size_t)prob->B * halves_bytes(prob, op));
-    *bytes += table16_bytes(prob);
   }
+  *bytes += table16_bytes(prob);
   return BCJR_OK;
 }
 
@@ -835,9 +858,6 @@ int bcjr_viterbi(const bcjr_problem* prob, const float* seq, const float* codebo
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
   if (packed && 8 % (prob->k * prob->V) != 0) return fail(BCJR_EINVAL, "packing needs k*V to divide 8");
-  Plan pl;
-  int rc = make_plan(prob, OP_VIT, &pl);
-  if (rc) return rc;
   bcjr::VitParams P = {};
   P.seq = seq;
   P.table = codebook_or_lut;
@@ -847,12 +867,11 @@ int bcjr_viterbi(const bcjr_problem* prob, const float* seq, const float* codebo
   P.recon = recon;
   P.mse = mse;
   P.packed = packed;
-  P.ws = static_cast<uint8_t*>(ws);
   P.B = prob->B;
   P.N = (int)prob->N;
   P.L = prob->L;
   P.Q = prob->Q;
-  return launch(pl, prob->B, ws_bytes, &P, stream);
+  return launch_viterbi(prob, P, ws, ws_bytes, stream);
 }
 
 int bcjr_viterbi_constrained(const bcjr_problem* prob, const float* seq, const float* codebook_or_lut,
@@ -868,9 +887,6 @@ int bcjr_viterbi_constrained(const bcjr_problem* prob, const float* seq, const f
   if (prob->code != BCJR_CODE_1MAD && prob->code != BCJR_CODE_3INST && !codebook_or_lut)
     return fail(BCJR_EINVAL, "code %d needs a codebook/LUT pointer", prob->code);
   if (packed && 8 % (prob->k * prob->V) != 0) return fail(BCJR_EINVAL, "packing needs k*V to divide 8");
-  Plan pl;
-  int rc = make_plan(prob, OP_VIT, &pl);
-  if (rc) return rc;
   bcjr::VitParams P = {};
   P.seq = seq;
   P.table = codebook_or_lut;
@@ -880,14 +896,13 @@ int bcjr_viterbi_constrained(const bcjr_problem* prob, const float* seq, const f
   P.recon = recon;
   P.mse = mse;
   P.packed = packed;
-  P.ws = static_cast<uint8_t*>(ws);
   P.overlap = overlap;
   P.overlap_bits = overlap_bits;
   P.B = prob->B;
   P.N = (int)prob->N;
   P.L = prob->L;
   P.Q = prob->Q;
-  return launch(pl, prob->B, ws_bytes, &P, stream);
+  return launch_viterbi(prob, P, ws, ws_bytes, stream);
 }
 
 int bcjr_decode(const bcjr_problem* prob, const int32_t* bitstream, const uint8_t* packed,

@@ -33,6 +33,22 @@ __device__ __forceinline__ bool vi_less(float a, int ia, float b, int ib) {
   return (a < b) || (a == b && ia < ib);
 }
 
+// A branch's cost and its index p as one double: the cost's bits above, p below.
+// Costs are >= 0, so doubles order the pairs by (cost, p), and one v_min_f64 per
+// branch keeps the smaller cost and, on a tie, the lower p.  (A float's bits in
+// the upper word are never a double's infinity or NaN for costs up to infinity,
+// and a cost of 0 gives a double denormal, which v_min_f64 keeps.)  The state loop
+// is bound by VALU issue; against a compare and two selects per branch, and the
+// wait states between them, per 4,096 sequences: 3INST N = 256 9.44 -> 7.9-8.0 ms
+// (74 instead of 93 VALU per 16-state butterfly), HYB column walk N = 128 5.74 ->
+// 4.34 ms (154 instead of 251 per 64 states).
+typedef float vit_pair __attribute__((ext_vector_type(2)));  // (p's bits, cost)
+__device__ __forceinline__ vit_pair vit_min(vit_pair a, vit_pair b) {
+  vit_pair r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // MAXT is the largest workgroup the instance is built for: 1024 threads (four
 // waves per SIMD, at most 128 VGPRs) where the codeword cache fits that budget,
 // else 512.
@@ -44,6 +60,7 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
   // Backpointers: kV bits per reduced state when a thread's RO outputs fill a
   // whole byte or half-word (kV = 2, 4), else one byte per state.
   constexpr bool PACK = RO * KV == 8 || RO * KV == 16;
+  constexpr bool kTab16 = CODE == CODE_TABLE && KV == 4;
   static_assert(!CACHE || NSUB == 1, "codeword cache needs whole butterflies per thread");
 
   extern __shared__ __align__(16) unsigned char smem[];
@@ -159,11 +176,21 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
   // the instance runs 1024 threads), held for the launch.
   const float2 cv_own = kColV ? col_entry(min(tid, 16 * 64 - 1)) : make_float2(0.0f, 0.0f);
 
+  float pid[R];  // p's bits, opaque: held, not formed again for every branch
+#pragma unroll
+  for (int p = 0; p < R; ++p) pid[p] = __builtin_bit_cast(float, opaque(p));
+
   const int row_bytes = PACK ? (NT * KV) >> 3 : NT;  // backpointer bytes per step
   for (long long b = blockIdx.x; b < P.B; b += gridDim.x) {
     uint8_t* bp = P.ws + (size_t)blockIdx.x * (size_t)N * (size_t)NT;
     const float* seqb = P.seq + (size_t)b * N * V;
-    for (int i = tid; i < N * V; i += nthr) wbuf[i] = seqb[i];
+    // A NaN weight enters the recursion as an infinity: every cost of its step and
+    // after is then infinite, so ties give the lowest branch and state, as costs of
+    // NaN (which compare false) do; the MSE reads the weights themselves.
+    for (int i = tid; i < N * V; i += nthr) {
+      const float w = seqb[i];
+      wbuf[i] = w == w ? w : INFINITY;
+    }
     // cum_{-1}, the vector step 0 reads: 0, or for a constrained sequence
     // kVitInf where the top ob bits of the step-0 state differ from ov.  Those
     // bits lie in s_0 >> kV (ob <= L - kV), so kVitInf + E_0(s) = kVitInf is the
@@ -219,7 +246,14 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
 #pragma unroll
           for (int p = 0; p < R; ++p) ri[p] = prev[p * NB + u];
           float ro[RO];
-          uint32_t bpw = 0;
+          uint32_t bi[RO];  // the outputs' best branches
+          // kV = 4 tables: codeword (p, output) of butterfly u at p NT + output SC + u SU
+          // of tab16, SC and SU those of the transposed copy (a wave's lanes, which
+          // hold consecutive u, then read consecutive addresses) or of the table.
+          // L = 16, V = 2, N = 128, 4,096 sequences: 74.6 ms in the table's order with
+          // compares, 16.0 ms with the copy.
+          const uint32_t SC_s = kTab16 ? opaque_uniform(P.SC) : 0u;
+          const uint32_t tl = kTab16 ? 4u * V * ((uint32_t)u * P.SU + (uint32_t)(sub * RO) * SC_s) : 0u;
           // The column walk's row step of output sub4 + r depends on it mod 8
           // (hyb_col_step), so each wave takes one of two unrolled copies
           // (sub4 mod 8 = SO, 0 or 4) whose cost reads are base + immediate.
@@ -228,8 +262,7 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
 #pragma unroll
             for (int r = 0; r < RO; ++r) {
               const int rr = sub * RO + r;
-              float best = 0.0f;
-              int bi = 0;
+              vit_pair best;
               const uint32_t ebase = kColV ? (cbv[r] >> 1) + eoff : 0u;  // table byte of output r's row-0 entry
 #pragma unroll
               for (int p = 0; p < R; ++p) {
@@ -241,6 +274,11 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
                   if constexpr (CACHE) {
 #pragma unroll
                     for (int v = 0; v < V; ++v) c[v] = cw[i][p][r][v];
+                  } else if constexpr (kTab16) {
+                    const char* row = reinterpret_cast<const char*>(P.tab16 + V * ((uint32_t)(p * NT) + (uint32_t)r * SC_s));
+                    const float* src = reinterpret_cast<const float*>(row + tl);
+#pragma unroll
+                    for (int v = 0; v < V; ++v) c[v] = src[v];
                   } else {
                     cword((uint32_t)(p * NT + R * u + rr), c);
                   }
@@ -251,14 +289,13 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
                     e = e + d2;
                   }
                 }
-                const float cum = ri[p] + e;
-                if (p == 0 || cum < best) {
-                  best = cum;
-                  bi = p;
-                }
+                vit_pair cand;
+                cand.x = pid[p];
+                cand.y = ri[p] + e;
+                best = p ? vit_min(best, cand) : cand;
               }
-              ro[r] = best;
-              bpw |= (uint32_t)bi << (8 * r);
+              ro[r] = best.y;
+              bi[r] = __builtin_bit_cast(uint32_t, (float)best.x);
             }
           };
           if (kColV && (sub4 & 4)) {
@@ -270,7 +307,7 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
           if constexpr (PACK) {  // entries R*u + sub*RO .. +RO-1 at kV bits each
             uint32_t bits = 0;
 #pragma unroll
-            for (int r = 0; r < RO; ++r) bits |= ((bpw >> (8 * r)) & (R - 1)) << (r * KV);
+            for (int r = 0; r < RO; ++r) bits |= bi[r] << (r * KV);
             uint8_t* row = bp + (size_t)t * row_bytes;
             const int e0 = R * u + sub * RO;
             if constexpr (RO * KV == 8) {
@@ -281,7 +318,7 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
           } else {
             uint8_t* bdst = bp + (size_t)t * NT + R * u + sub * RO;
 #pragma unroll
-            for (int r = 0; r < RO; ++r) bdst[r] = (uint8_t)(bpw >> (8 * r));
+            for (int r = 0; r < RO; ++r) bdst[r] = (uint8_t)bi[r];
           }
         }
       }
@@ -400,7 +437,7 @@ __global__ __launch_bounds__(MAXT) void bcjr_viterbi_kernel(VitParams P) {
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         if (P.recon) P.recon[((size_t)b * N + t) * V + v] = c[v];
-        const double d = (double)c[v] - (double)wbuf[t * V + v];
+        const double d = (double)c[v] - (double)seqb[t * V + v];
         se += d * d;
       }
     }

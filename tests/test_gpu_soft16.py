@@ -175,3 +175,38 @@ def test_sequences_beside_each_other_in_two_halves(bcjr_mod, oracle, B):
     rows = [0, 64, B - 1]
     assert _rel(soft.cpu().numpy()[rows], oracle.bcjr_forward(x[rows], cb.cpu().numpy(), T, L, 2)[0]) < SOFT_TOL
     assert _rel(d.cpu().numpy()[rows], oracle.bcjr_backward(x[rows], cb.cpu().numpy(), T, L, 2, g[rows])) < GRAD_TOL
+
+
+@pytest.mark.parametrize("L,k,V,N", [(16, 2, 2, 9), (14, 2, 2, 6), (9, 4, 1, 5)])
+def test_viterbi_table_with_and_without_its_copy(bcjr_mod, oracle, L, k, V, N):
+    """kV = 4 tables: the full workspace (transposed copy) and one slot (the table
+    as it is) give the oracle's walks, with ties (a table of few values), a NaN
+    and an infinite weight among the sequences."""
+    from bcjr import _lib
+    lib = _lib.load()
+    B = 5
+    rng = np.random.default_rng(L)
+    cb_np = np.round(2 * rng.standard_normal((1 << L, V))).astype(np.float32) / 2
+    x = np.round(rng.standard_normal((B, N, V)) * 4).astype(np.float32) / 4
+    x[3, 1, 0], x[4, 2, V - 1] = np.nan, np.inf
+    cb, xd = torch.tensor(cb_np, device="cuda"), torch.tensor(x, device="cuda")
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, k, V, torch.device("cuda"))
+    prob = spec.problem(B, N)
+    full = ctypes.c_size_t(0)
+    _lib.check(lib.bcjr_workspace_bytes(ctypes.byref(prob), 2, ctypes.byref(full)), "ws")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    walk_ref = oracle.viterbi(x[:3], cb_np, L, 4)[0]
+    slot = (N * (1 << (L - 4)) + 255) // 256 * 256
+    res = []
+    for nbytes in (full.value, slot):
+        print(f"[viterbi] table L={L} k={k} V={V} workspace {nbytes}", flush=True)
+        ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device="cuda")
+        walk = torch.full((B, N), -1, dtype=torch.int32, device="cuda")
+        mse = torch.zeros(B, device="cuda")
+        _lib.check(lib.bcjr_viterbi(ctypes.byref(prob), xd.data_ptr(), _lib.ptr(table), walk.data_ptr(), None, None, None,
+                                    mse.data_ptr(), None, ws.data_ptr(), nbytes, stream), "viterbi")
+        torch.cuda.synchronize()
+        assert np.array_equal(walk.cpu().numpy()[:3], walk_ref)
+        assert torch.isnan(mse[3]) and torch.isinf(mse[4])
+        res.append(walk.cpu().numpy())
+    assert np.array_equal(res[0], res[1]) and res[0].min() >= 0 and res[0].max() < 1 << L
