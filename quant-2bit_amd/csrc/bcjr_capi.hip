@@ -644,10 +644,10 @@ int rht_impl(const float* W, float* out, int64_t batch, int64_t m, int64_t n, co
   // inverse: rows of W H_n then diag(sr), then H_m, row signs and the scale.
   if (n >= 64 && aligned16(W) && aligned16(sign_r)) {  // tiled kernels: 2 passes over HBM for most shapes
     hipError_t e = inverse
-        ? bcjr::launch_fwht_tiled(W, out, (int)batch, (int)m, (int)n, true, nullptr, sign_r, nullptr, sign_l, s,
-                                  di.num_cu * 4, stream)
-        : bcjr::launch_fwht_tiled(W, out, (int)batch, (int)m, (int)n, true, sign_r, nullptr, sign_l, nullptr, s,
-                                  di.num_cu * 4, stream);
+        ? bcjr::launch_fwht_tiled(W, out, (int)batch, (int)m, (int)n, true, nullptr, nullptr, sign_r, sign_l, s,
+                                  stream)
+        : bcjr::launch_fwht_tiled(W, out, (int)batch, (int)m, (int)n, true, sign_r, sign_l, nullptr, nullptr, s,
+                                  stream);
     return e == hipSuccess ? BCJR_OK : hip_fail(e, "bcjr_rht tiled passes");
   }
   hipError_t e =
@@ -1048,7 +1048,7 @@ int bcjr_hadamard(const float* x, float* out, int64_t rows, int64_t n, float sca
   hipError_t e;
   if (n >= 64 && rows <= INT32_MAX && aligned16(x))
     e = bcjr::launch_fwht_tiled(x, out, 1, (int)rows, (int)n, false, nullptr, nullptr, nullptr, nullptr, scale,
-                                di.num_cu * 4, stream);
+                                stream);
   else
     e = bcjr::launch_fwht_rows(x, out, rows, (int)n, nullptr, nullptr, rows, nullptr, scale, di.num_cu * 8, stream);
   return e == hipSuccess ? BCJR_OK : hip_fail(e, "bcjr_hadamard launch");

@@ -80,9 +80,9 @@ hipError_t launch_fwht_rows(const float* x, float* out, long long rows, int n, c
                             int max_blocks, hipStream_t stream);
 hipError_t launch_fwht_cols(float* x, int batch, int m, int n, const float* row_sign, float scale,
                             int max_blocks, hipStream_t stream);
-hipError_t launch_fwht_tiled(const float* x, float* out, int batch, int m, int n, bool col, const float* pre,
-                             const float* post, const float* row_mid, const float* row_end, float scale,
-                             int max_blocks, hipStream_t stream);
+hipError_t launch_fwht_tiled(const float* x, float* out, int batch, int m, int n, bool col, const float* pre_col,
+                             const float* pre_row, const float* post_col, const float* post_row, float scale,
+                             hipStream_t stream);
 
 // The kernel-side code of a soft launch, or of a 1024-thread Viterbi launch:
 // HYB at L = 16, kV = 4, 3 <= Q <= 9 takes the column-walk LUT (code 4,
