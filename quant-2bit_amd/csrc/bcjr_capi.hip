@@ -442,8 +442,6 @@ int launch(const Plan& pl, long long B, size_t ws_bytes, void* params, hipStream
   return BCJR_OK;
 }
 
-}  // namespace
-
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Bytes the two-halves launches keep per sequence: its slot, the two state
@@ -591,6 +589,8 @@ int launch_soft(const bcjr_problem* p, int op, bcjr::Soft16Params P, void* ws, s
   P.B = p->B;
   return launch(pl, p->B, left, &P, stream);
 }
+
+}  // namespace
 
 // Sequence slots of bcjr_forward_noalloc: a static device array, one copy per
 // GPU.  Host code never names it after set-up: its host-side symbol is only a

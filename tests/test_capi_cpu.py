@@ -44,6 +44,15 @@ def test_library_exports_every_declared_symbol(lib):
         assert re.search(rf"\bT {name}\b", out), name
 
 
+def test_library_exports_no_global_names_of_its_own(lib):
+    """Outside the C ABI and namespace bcjr the library defines no dynamic symbol
+    that another library's function of the same name could take the place of."""
+    names = [ln.split() for ln in os.popen(f"nm -D --defined-only {lib._name}").read().splitlines()]
+    ours = set(_declared_functions())
+    stray = [n[-1] for n in names if n[-2] == "T" and n[-1] not in ours and not n[-1].startswith("_ZN4bcjr")]
+    assert not stray, stray
+
+
 def test_strerror_and_version(lib):
     assert lib.bcjr_version().startswith(b"bcjr_hip")
     assert lib.bcjr_strerror(0) == b"ok"
