@@ -70,6 +70,7 @@ struct Plan {
   int NT = 0, NB = 0, NU = 0;
   int nthr = 0, upt = 0;
   bool cache = false;
+  bool fits = true;  // two-halves plans: there is a kernel and the LDS holds its state
   const void* fn = nullptr;
   size_t lds = 0;
   size_t slot_bytes = 0;
@@ -153,7 +154,7 @@ struct PlanKey {
            Q == o.Q && wide == o.wide && N == o.N;
   }
 };
-constexpr int kPlanCache = 64;
+constexpr int kPlanCache = 128;  // a problem has up to two plans per operation
 std::mutex g_plan_mu;
 PlanKey g_plan_keys[kPlanCache];
 Plan g_plans[kPlanCache];
@@ -273,6 +274,19 @@ bcjr::Swizzle pick_swizzle(int L, int KV) {
   return best;
 }
 
+// The search takes up to 55 ms (L = 15): once per (L, kV).
+bcjr::Swizzle swizzle_of(int L, int KV) {
+  static std::mutex mu;
+  static bool have[17][5];
+  static bcjr::Swizzle memo[17][5];
+  std::lock_guard<std::mutex> lk(mu);
+  if (!have[L][KV]) {
+    memo[L][KV] = pick_swizzle(L, KV);
+    have[L][KV] = true;
+  }
+  return memo[L][KV];
+}
+
 // State layout of the column-walk backward instance (L = 16, kV = 4), whose
 // thread tid holds butterfly col_walk_unit(tid) rather than tid: with this
 // swizzle every half-wave's 64-bit reads and every quarter-wave's 64-bit writes
@@ -316,7 +330,7 @@ int make_soft16_plan(const bcjr_problem* p, int op, bool wide, const DeviceInfo&
   pl->nthr = (pl->NB + per_wave - 1) / per_wave * 64;
   pl->fn = bcjr::soft16_kernel_ptr(kind, p->V, code, lpb);
   pl->lds = bcjr::soft16_lds_bytes(p->L, p->V, (int)p->N, pl->nthr / 64, code, p->Q, kind);
-  pl->swz = code == bcjr::CODE_HYB_COL ? kColWalkSwizzle : pick_swizzle(p->L, 4);
+  pl->swz = code == bcjr::CODE_HYB_COL ? kColWalkSwizzle : swizzle_of(p->L, 4);
   pl->slot_bytes = slot_bytes_of(p, op == OP_BWD ? OP_BWD : OP_FWD);
   return finish_plan(p, di, pl);
 }
@@ -326,22 +340,33 @@ int make_soft16_plan(const bcjr_problem* p, int op, bool wide, const DeviceInfo&
 // and backward, whole butterflies against a lane per output: L = 13, 128 sequences
 // 0.28 against 0.37 and 0.41 against 0.49 ms; L = 12 0.24 against 0.27 and 0.32
 // against 0.32 ms; L = 10, 64 sequences 0.21 against 0.18 and 0.26 against 0.21 ms).
+struct HalvesShape {
+  int lpb, upt, nthr;
+};
+
+HalvesShape halves_shape(const bcjr_problem* p) {
+  const int KV = p->k * p->V, NB = 1 << (p->L - 2 * KV), lpb = KV == 2 && p->L >= 12 ? 1 : 1 << KV;
+  const int upt = std::max(1, NB * lpb / 1024);
+  return {lpb, upt, std::max(64, NB * lpb / upt)};
+}
+
 int make_halves_plan(const bcjr_problem* p, int op, const DeviceInfo& di, Plan* pl) {
   const int KV = p->k * p->V, kind = op == OP_BWD ? 1 : op == OP_FWD_ENTROPY ? 2 : 0;
-  const int lpb = KV == 2 && p->L >= 12 ? 1 : 1 << KV;
+  const HalvesShape sh = halves_shape(p);
+  const bool in_place = bcjr::halves_in_place(op == OP_BWD, sh.upt, sh.lpb);
   pl->KV = KV;
   pl->R = 1 << KV;
   pl->NSUB = 1;
   pl->NT = 1 << (p->L - KV);
   pl->NB = pl->NT >> KV;
   pl->NU = pl->NB;
-  pl->upt = std::max(1, pl->NB * lpb / 1024);
-  pl->nthr = std::max(64, pl->NB * lpb / pl->upt);
-  pl->fn = bcjr::halves_kernel_ptr(kind, KV, p->V, p->code, pl->upt, lpb);
-  if (!pl->fn) return fail(BCJR_EUNSUPPORTED, "no two-halves kernel for L=%d k=%d V=%d code=%d", p->L, p->k, p->V, p->code);
-  pl->lds = bcjr::halves_lds_bytes(p->L, KV, p->V, (int)p->N, pl->nthr / 64, p->code, p->Q, kind,
-                                   bcjr::halves_in_place(op == OP_BWD, pl->upt, lpb));
-  pl->swz = pick_swizzle(p->L, KV);
+  pl->upt = sh.upt;
+  pl->nthr = sh.nthr;
+  pl->fn = bcjr::halves_kernel_ptr(kind, KV, p->V, p->code, sh.upt, sh.lpb);
+  pl->lds = bcjr::halves_lds_bytes(p->L, KV, p->V, (int)p->N, pl->nthr / 64, p->code, p->Q, kind, in_place);
+  pl->fits = pl->fn && pl->lds <= di.max_lds;  // long N (or large Q): a plan like any other, kept as "no"
+  if (!pl->fits) return BCJR_OK;
+  if (in_place) pl->swz = swizzle_of(p->L, KV);
   pl->slot_bytes = slot_bytes_of(p, op == OP_BWD ? OP_BWD : OP_FWD);
   return finish_plan(p, di, pl);
 }
@@ -416,7 +441,7 @@ int make_plan_uncached(const bcjr_problem* p, int op, bool wide, const DeviceInf
     pl->slot_bytes = slot_bytes_of(p, fwd ? OP_FWD : OP_VIT);
   } else {
     pl->cache = false;
-    pl->swz = pick_swizzle(p->L, KV);
+    pl->swz = swizzle_of(p->L, KV);
     pl->fn = bcjr::bwd_kernel_ptr(KV, p->V, kcode, upt);
     pl->lds = bcjr::bwd_lds_bytes(p->L, KV, p->V, N, nwaves, kcode, p->Q);
     pl->slot_bytes = slot_bytes_of(p, OP_BWD);
@@ -474,9 +499,10 @@ int halves_plan(const bcjr_problem* p, int op, const Plan& pl, Plan* out, bool* 
       return make_plan(p, op, out, true);
     return BCJR_OK;
   }
+  // no plan is made for a batch that 32 waves a CU could not hold
+  if (2 * p->B > (long long)pl.num_cu * (2048 / halves_shape(p).nthr)) return BCJR_OK;
   const int rc = make_plan(p, op, out, true);
-  if (rc == BCJR_EUNSUPPORTED) return BCJR_OK;  // its LDS does not hold this N (or Q): one launch
-  if (rc) return rc;
+  if (rc || !out->fits) return rc;  // the LDS does not hold this N (or Q): one launch
   *halves = 2 * p->B <= out->max_blocks;
   return BCJR_OK;
 }
