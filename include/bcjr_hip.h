@@ -162,6 +162,8 @@ int bcjr_backward(const bcjr_problem* prob, const float* seq, const float* T,
  *   mse (B,) float32 mean squared error of recon vs seq,
  *   packed (B, ceil(N*kV/8)) uint8: bitstream packed LSB-first, step t in
  *   bits [t*kV, (t+1)*kV).
+ * A NaN codeword counts as an infinite cost, as does a NaN weight (every cost of
+ * its sequence is then infinite; its walk is a walk of the trellis, no more).
  * Replaces viterbi_encode_v_batched_cuda (src/viterbi/cuda_kernel.py:166-220). */
 int bcjr_viterbi(const bcjr_problem* prob, const float* seq, const float* codebook_or_lut,
                  int32_t* walk, int32_t* bitstream, int32_t* start_state, float* recon,

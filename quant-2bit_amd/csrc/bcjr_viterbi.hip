@@ -37,7 +37,10 @@ __device__ __forceinline__ bool vi_less(float a, int ia, float b, int ib) {
 // Costs are >= 0, so doubles order the pairs by (cost, p), and one v_min_f64 per
 // branch keeps the smaller cost and, on a tie, the lower p.  (A float's bits in
 // the upper word are never a double's infinity or NaN for costs up to infinity,
-// and a cost of 0 gives a double denormal, which v_min_f64 keeps.)  The state loop
+// and a cost of 0 gives a double denormal, which v_min_f64 keeps.)  A codeword that
+// is NaN (a table's or LUT's) makes its costs NaN, of either sign; the candidates
+// enter by their absolute value, an operand modifier, so that such a branch comes
+// after every other, infinite ones included.  The state loop
 // is bound by VALU issue; against a compare and two selects per branch, and the
 // wait states between them, per 4,096 sequences: 3INST N = 256 9.44 -> 7.9-8.0 ms
 // (74 instead of 93 VALU per 16-state butterfly), HYB column walk N = 128 5.74 ->
@@ -45,7 +48,7 @@ __device__ __forceinline__ bool vi_less(float a, int ia, float b, int ib) {
 typedef float vit_pair __attribute__((ext_vector_type(2)));  // (p's bits, cost)
 __device__ __forceinline__ vit_pair vit_min(vit_pair a, vit_pair b) {
   vit_pair r;
-  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
   return r;
 }
 

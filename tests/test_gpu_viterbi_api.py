@@ -240,3 +240,36 @@ def test_return_trace_api_and_reference_gate_shape(bcjr_mod, oracle):
     t_r, b_r = oracle.viterbi_trace(seq2.reshape(128, 2), cbh, 16, 4)
     assert np.array_equal(out[4], t_r) and np.array_equal(out[5], b_r)
     assert int(np.argmin(out[4][-1])) == int(np.argmin(t_r[-1]))
+
+
+@pytest.mark.parametrize("L,k,V,kind", [(8, 1, 1, "table"), (10, 2, 1, "table"), (16, 2, 1, "table"), (12, 1, 2, "table"),
+                                        (15, 1, 2, "table"), (9, 4, 1, "table"), (14, 4, 1, "table"), (10, 2, 2, "table"),
+                                        (16, 2, 2, "table"), (10, 2, 2, "hyb"), (16, 2, 2, "hyb"), (13, 1, 2, "hyb")])
+def test_codewords_that_are_not_finite(bcjr_mod, oracle, L, k, V, kind):
+    """NaN of both signs and infinities among the codewords count as an infinite
+    cost, as a NaN weight does: the walk of a finite sequence is that of the
+    codebook with infinities in their place.  A sequence with a NaN or an infinite
+    weight costs infinity everywhere; its walk stays in the trellis."""
+    from bcjr import ops
+    print(f"[viterbi] {kind} L={L} k={k} V={V}, codewords that are not finite", flush=True)
+    rng = np.random.default_rng(100 * L + k)
+    odd = np.array([0x7FC00000, 0xFFC00000, 0x7F800000, 0xFF800000], np.uint32).view(np.float32)
+    tab = np.round(4 * rng.standard_normal((512, 2) if kind == "hyb" else (1 << L, V))).astype(np.float32) / 4
+    flat = tab.reshape(-1)
+    at = 8 + rng.choice(flat.size - 8, max(4, flat.size // 50), replace=False)
+    flat[at] = odd[np.arange(at.size) % 4]
+    if kind == "hyb":
+        cb = bcjr_mod.make_hyb_codebook_gpu(tab, 9, L, "cuda")
+    else:
+        cb = torch.tensor(tab, device="cuda")
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, k, V, torch.device("cuda"))
+    B, N = 7, 9
+    x = np.round(4 * rng.standard_normal((B, N, V))).astype(np.float32) / 4
+    x[4, 3, 0], x[5, 2, V - 1], x[6, 8, 0] = np.nan, np.inf, -np.inf
+    walk = ops.viterbi(spec, torch.tensor(x, device="cuda"), table)["walk"]
+    cb_inf = cb.cpu().numpy()
+    cb_inf = np.where(np.isnan(cb_inf), np.float32(np.inf), cb_inf)
+    walk = walk.cpu().numpy()
+    assert np.array_equal(walk[:4], oracle.viterbi(x[:4], cb_inf, L, k * V)[0])
+    assert np.isfinite(cb_inf[walk[:4]]).all()
+    assert walk.min() >= 0 and walk.max() < 1 << L
