@@ -98,7 +98,13 @@ typedef struct {
 
 /* Bytes of device workspace the operation wants for this problem on the
  * current device.  A smaller buffer (>= one sequence slot) also works, with
- * fewer sequences in flight. */
+ * fewer sequences in flight.
+ *
+ * A soft call on a batch that leaves half of the chip idle runs every sequence
+ * in two halves, which sum in another order than one launch does: a sequence's
+ * result can differ in its last bits with the size of the batch it is in (and
+ * the operation: forward, entropy and backward switch at different sizes), and
+ * with a workspace too short for the halves.  Equal calls give equal bits. */
 int bcjr_workspace_bytes(const bcjr_problem* prob, int op, size_t* bytes);
 
 /* Soft codewords E_P[c(s_t)] (B, N, V) and log Z (B,) (natural log, including
@@ -132,9 +138,11 @@ int bcjr_forward_entropy(const bcjr_problem* prob, const float* seq, const float
  * counterpart in the reference; it is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  The sequence slots live in a static device array of
- * BCJR_NOALLOC_SCRATCH_BYTES (128 MiB) that the library holds on every GPU it
- * runs on until the process ends; as many sequences are in flight as slots fit
- * (8 at L=16, kV=2, N=256), so its throughput is below bcjr_forward's.  A
+ * BCJR_NOALLOC_SCRATCH_BYTES (128 MiB; and 17 MiB for the state of batches in
+ * two halves) that the library holds on every GPU it runs on until the process
+ * ends; as many sequences are in flight as slots fit (8 at L=16, kV=2, N=256),
+ * so its throughput is below bcjr_forward's.  With 2^(L-kV) >= 32 its results
+ * are bcjr_forward's bit for bit.  A
  * problem whose one slot (N * 2^(L-kV) * 4 bytes) exceeds the array returns
  * BCJR_EWORKSPACE.  Every call on a GPU shares that GPU's array: calls that
  * overlap on one GPU (other streams, other threads) race and must be

@@ -480,9 +480,10 @@ size_t halves_bytes(const bcjr_problem* p, int op) {
 // Whether a soft call runs its sequences in two halves each (bcjr_soft16.h,
 // bcjr_halves.h), and on which plan: when twice as many workgroups still all fit
 // at once, so that the steps in sequence are halved and no sequence waits for
-// another.  The choice depends on the problem and the device only, not on the
-// workspace (a short one takes several rounds), so every workspace gives the same
-// bits.  kV = 4: the plan of one launch, or, column walk, one workgroup of twice
+// another.  A sequence's last bits therefore depend on the batch it is in: the two
+// forms sum in other orders.  Every workspace of the queried size, and every
+// shorter one that takes several rounds, gives the same bits; one too short for
+// that (launch_halves) runs in one launch, with the bits of a large batch.  kV = 4: the plan of one launch, or, column walk, one workgroup of twice
 // the threads per CU where that is all there is.
 // Measured, forward and backward, one launch -> two halves, N = 128: column walk
 // 8 sequences 1.17 -> 0.62 and 1.83 -> 0.85 ms (narrow workgroup 0.70 and 1.01),
@@ -535,13 +536,20 @@ int launch_viterbi(const bcjr_problem* p, bcjr::VitParams P, void* ws, size_t ws
   return launch(pl, p->B, ws_bytes, &P, stream);
 }
 
-// The two launches of a batch in two halves, over as many sequences a round as the
-// workspace holds; *done = false when it does not hold one.
-int launch_halves(const bcjr_problem* p, int op, const Plan& pl, bcjr::Soft16Params P, char* ws, size_t ws_bytes,
-                  hipStream_t stream, bool* done) {
-  const long long round = std::min<long long>(p->B, (long long)(ws_bytes / halves_bytes(p, op)));
-  *done = round >= 1;
-  if (!*done) return BCJR_OK;
+// The two launches of a batch in two halves; a workspace that does not hold all of
+// it takes equal rounds.  *done = false where one launch (plan `one`) is the better
+// use of a short workspace: N steps in series a round against 2 N for as many
+// sequences as it has slots for, or no room for one sequence's halves.
+int launch_halves(const bcjr_problem* p, int op, const Plan& one, const Plan& pl, bcjr::Soft16Params P, char* ws,
+                  size_t ws_bytes, hipStream_t stream, bool* done) {
+  const long long fit = (long long)(ws_bytes / halves_bytes(p, op));
+  *done = false;
+  if (fit < 1) return BCJR_OK;
+  const long long flight = std::min<long long>(one.max_blocks, (long long)(ws_bytes / one.slot_bytes));
+  const long long rounds = (p->B + fit - 1) / fit;
+  if (rounds >= 2 * ((p->B + flight - 1) / flight)) return BCJR_OK;
+  const long long round = (p->B + rounds - 1) / rounds;
+  *done = true;
   const size_t st = op == OP_BWD ? 2 : 1, row = (size_t)p->N * p->V;
   char* mid = ws + (size_t)round * pl.slot_bytes;
   P.ws = reinterpret_cast<float*>(ws);
@@ -604,7 +612,7 @@ int launch_soft(const bcjr_problem* p, int op, bcjr::Soft16Params P, void* ws, s
   P.t_per_seq = p->t_per_seq ? 1 : 0;
   P.slot_floats = pl.slot_bytes / sizeof(float);
   if (halves) {
-    rc = launch_halves(p, op, hp, P, w, left, stream, done);
+    rc = launch_halves(p, op, pl, hp, P, w, left, stream, done);
     if (rc || *done) return rc;
   }
   if (pl.KV != 4) return BCJR_OK;
@@ -622,7 +630,12 @@ int launch_soft(const bcjr_problem* p, int op, bcjr::Soft16Params P, void* ws, s
 // GPU.  Host code never names it after set-up: its host-side symbol is only a
 // stand-in, so the device address comes from hipGetSymbolAddress, once per
 // device with that device current, and is kept per device.
-static __device__ __align__(256) unsigned char scratch[BCJR_NOALLOC_SCRATCH_BYTES];
+// The slots are followed by room for what a batch in two halves keeps beside them
+// (halves_bytes): 128 KiB and 8 (N + 2) bytes a sequence at L = 16, kV = 2, so a
+// batch whose slots fit runs as bcjr_forward runs it (from 2^(L-kV) = 32 on: the
+// offsets of a smaller trellis are as large as its slots).
+constexpr size_t kNoallocBytes = BCJR_NOALLOC_SCRATCH_BYTES + ((size_t)17 << 20);
+static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 
 namespace {
 
@@ -753,7 +766,7 @@ int bcjr_forward_noalloc(const bcjr_problem* prob, const float* seq, const float
   void* ws = nullptr;
   rc = scratch_ptr(&ws);
   if (rc) return rc;
-  return bcjr_forward(prob, seq, T, codebook_or_lut, soft, logZ, ws, BCJR_NOALLOC_SCRATCH_BYTES, stream);
+  return bcjr_forward(prob, seq, T, codebook_or_lut, soft, logZ, ws, kNoallocBytes, stream);
 }
 
 int bcjr_forward_internals(const bcjr_problem* prob, const float* seq, const float* T,

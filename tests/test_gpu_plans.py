@@ -59,3 +59,118 @@ def test_shape_whose_halves_do_not_fit_is_planned_once(bcjr_mod, oracle):
     d = ops.backward(spec, torch.tensor(x, device="cuda"), 0.2, table, torch.tensor(g, device="cuda"))
     ref = oracle.bcjr_backward(x, cb.cpu().numpy(), 0.2, L, 2, g)
     assert max_rel(d.cpu().numpy(), ref) < 1e-3  # the parity bound of the gradient
+
+
+def _codebook(bcjr, kind, L, V):
+    if kind == "hyb":
+        lut = np.random.default_rng(L).standard_normal((512, 2)).astype(np.float32)
+        return bcjr.make_hyb_codebook_gpu(lut, 9, L, "cuda")
+    if kind == "1mad":
+        return bcjr.make_1mad_codebook(L, "cuda")
+    return torch.tensor(np.random.default_rng(L).standard_normal((1 << L, V)).astype(np.float32), device="cuda")
+
+
+@pytest.mark.parametrize("op", ["forward", "entropy", "backward"])
+@pytest.mark.parametrize("kind,L,k,V,N", [("hyb", 16, 2, 2, 12), ("table", 16, 2, 2, 12), ("hyb", 12, 2, 2, 20),
+                                          ("1mad", 12, 2, 1, 24), ("1mad", 16, 2, 1, 16), ("table", 10, 1, 1, 32)])
+def test_rounds_of_a_short_workspace(bcjr_mod, kind, L, k, V, N, op):
+    """8 sequences (one of them NaN, each at its own T and g_logZ): a workspace for
+    3 of their halves gives every output of the full one bit for bit, in rounds of
+    3, 3 and 2; one of 8 slots, which 7 halves exhaust at most, runs one launch as
+    one slot does, bit for bit, and within the tolerances of the parity tests of
+    the halves."""
+    from bcjr import _lib
+    lib = _lib.load()
+    B, kV = 8, k * V
+    cb = _codebook(bcjr_mod, kind, L, V)
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, k, V, torch.device("cuda"))
+    rng = np.random.default_rng(L + N)
+    x, g = (rng.standard_normal((B, N, V)).astype(np.float32) for _ in range(2))
+    x[5, 3, 0] = np.nan
+    T = np.array([0.05, 0.1, 0.2, 0.06, 0.5, 0.1, 0.3, 0.07], np.float32)
+    gz = rng.standard_normal(B).astype(np.float32)
+    xd, gd, Td, gzd = (torch.tensor(a, device="cuda") for a in (x, g, T, gz))
+    prob = spec.problem(B, N, True)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    st, nt = (2 if op == "backward" else 1), 1 << (L - kV)
+    full = ctypes.c_size_t(0)
+    _lib.check(lib.bcjr_workspace_bytes(ctypes.byref(prob), 1 if op == "backward" else 0, ctypes.byref(full)), "ws")
+    up = lambda b: (b + 255) // 256 * 256
+    slot = up(N * nt * 4 * st)
+    halves = slot + up(2 * st * nt * 4) + up(8 * (N + 2))
+    copy = 4 * V << L if kind == "table" and kV == 4 else 0
+    assert full.value >= copy + B * halves and 8 * slot < 8 * halves
+    res = []
+    for nbytes in (full.value, copy + 3 * halves, copy + B * slot, copy + slot):
+        _say(f"{op} {kind} L={L} kV={kV}: workspace {nbytes}")
+        ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device="cuda")
+        out, z, H = (torch.full(s, 7.0, device="cuda") for s in ((B, N, V), (B,), (B, N)))
+        if op == "backward":
+            rc = lib.bcjr_backward(ctypes.byref(prob), xd.data_ptr(), Td.data_ptr(), _lib.ptr(table), None, gd.data_ptr(),
+                                   gzd.data_ptr(), out.data_ptr(), ws.data_ptr(), nbytes, stream)
+            got = [out]
+        elif op == "entropy":
+            rc = lib.bcjr_forward_entropy(ctypes.byref(prob), xd.data_ptr(), Td.data_ptr(), _lib.ptr(table), out.data_ptr(),
+                                          z.data_ptr(), H.data_ptr(), ws.data_ptr(), nbytes, stream)
+            got = [out, z, H]
+        else:
+            rc = lib.bcjr_forward(ctypes.byref(prob), xd.data_ptr(), Td.data_ptr(), _lib.ptr(table), out.data_ptr(),
+                                  z.data_ptr(), ws.data_ptr(), nbytes, stream)
+            got = [out, z]
+        _lib.check(rc, op)
+        torch.cuda.synchronize()
+        got = [t.cpu().numpy() for t in got]
+        for t in got:
+            assert np.isnan(t[5]).all() and np.isfinite(np.delete(t, 5, 0)).all()
+        res.append(got)
+    for a, b in zip(res[0], res[1]):
+        assert np.array_equal(a, b, equal_nan=True)
+    for a, b in zip(res[2], res[3]):
+        assert np.array_equal(a, b, equal_nan=True)
+    tol = [1e-3] if op == "backward" else [1e-4, 1e-5, 1e-4]  # gradient; soft, log Z, entropy: the parity tests' bounds
+    for a, b, t in zip(res[0], res[2], tol):
+        assert max_rel(np.delete(a, 5, 0), np.delete(b, 5, 0)) < t
+
+
+@pytest.mark.parametrize("N,B", [(2048, 1), (2048, 2), (256, 8)])
+def test_noalloc_holds_its_slots_in_two_halves(bcjr_mod, N, B):
+    """L = 16, kV = 2: one slot of 128 MiB, and eight of 16, run as bcjr_forward runs
+    them, bit for bit and (8 sequences) in one round: with seven halves in a round it
+    took two, about twice as long."""
+    from bcjr import _lib
+    lib = _lib.load()
+    L = 16
+    x = torch.randn(B, N, 1, device="cuda", generator=torch.Generator("cuda").manual_seed(N))
+    T = torch.full((1,), 0.1, device="cuda")
+    prob = _lib.Problem(L, 2, 1, B, N, _lib.CODE_3INST, 9, 0)
+    n = ctypes.c_size_t(0)
+    _lib.check(lib.bcjr_workspace_bytes(ctypes.byref(prob), 0, ctypes.byref(n)), "ws")
+    ws = torch.empty(n.value, dtype=torch.uint8, device="cuda")
+    out = [[torch.full_like(x, 7.0), torch.full((B,), 7.0, device="cuda")] for _ in range(2)]
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def run(i):
+        args = [ctypes.byref(prob), x.data_ptr(), T.data_ptr(), None, out[i][0].data_ptr(), out[i][1].data_ptr()]
+        _lib.check(lib.bcjr_forward_noalloc(*args, stream) if i else
+                   lib.bcjr_forward(*args, ws.data_ptr(), ws.numel(), stream), "forward")
+
+    def ms(i):
+        times = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            run(i)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    _say(f"noalloc N={N} B={B}")
+    run(0), run(1)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert torch.isfinite(out[1][0]).all()
+    if B == 8:
+        with_ws, without = ms(0), ms(1)
+        _say(f"8 sequences: {with_ws:.3f} ms with a workspace, {without:.3f} ms without")
+        assert without < 1.5 * with_ws
