@@ -33,10 +33,15 @@
 namespace bcjr {
 
 // Codewords of a lane kept in VGPRs over a sweep: all of them up to 64 values,
-// except in the backward's gradient-forming sweep past 16 and in the low-temperature
-// variant past 16, whose working sets need the registers.
-constexpr bool halves_cached(int values, bool grad_marg, bool exact) {
-  return values <= ((grad_marg || exact) ? 16 : 64);
+// except in the backward's gradient-forming sweep past 16 and in the computed
+// codes' low-temperature variant past 16, whose working sets need the registers.
+// A table's variant holds them there too, and unrolls its units where it does not,
+// so that their reads overlap: read one unit after the other, they cost more than
+// the halves save (T = 0.06, N = 96, 8 sequences, forward, backward, entropy:
+// L = 15 0.78, 0.83, 0.79 -> 0.26, 0.57, 0.28 ms, in one launch 0.56, 0.71, 0.52;
+// L = 16 1.46, 1.58, 1.46 -> 0.45, 1.03, 0.49, in one launch 1.03, 1.48, 1.55).
+constexpr bool halves_cached(int values, bool grad_marg, bool exact_computed) {
+  return values <= ((grad_marg || exact_computed) ? 16 : 64);
 }
 
 template <int KV, int V, int CODE, int UPT, int LPB, bool GRAD, bool ENT>
@@ -149,7 +154,7 @@ __global__ __launch_bounds__(1024, 4) void bcjr_halves_kernel(Soft16Params P) {
                    float O0) __attribute__((always_inline)) -> double {
     constexpr bool BETA = decltype(beta_tag)::value, MARG = decltype(marg_tag)::value;
     constexpr bool EXACT = decltype(exact_tag)::value;
-    constexpr bool CACHE = V == 1 && halves_cached(UPT * R * RO, GRAD && MARG, EXACT);
+    constexpr bool CACHE = V == 1 && halves_cached(UPT * R * RO, GRAD && MARG, EXACT && CODE != CODE_TABLE);
     constexpr int dt = BETA ? -1 : 1;
     const int o_lane = LPB == 1 ? 0 : part;
     // Codeword of output j + o_lane, input i of unit q: state p*NT + R*u + c with
@@ -216,8 +221,8 @@ __global__ __launch_bounds__(1024, 4) void bcjr_halves_kernel(Soft16Params P) {
 #pragma unroll
       for (int v = 0; v < NS; ++v) acc[v] = 0.0f;
       if (live) {
-        // One unit: unrolled, or in the low-temperature variant, which forms every
-        // codeword, a loop, so that one unit's registers serve all.
+        // One unit: unrolled, or in the low-temperature variant of the codes it computes,
+        // a loop, so that one unit's registers serve all.
         auto unit = [&](int q) __attribute__((always_inline)) {
           __builtin_amdgcn_sched_barrier(0);
           // (also keeps the hashes inside the step)
@@ -357,7 +362,7 @@ __global__ __launch_bounds__(1024, 4) void bcjr_halves_kernel(Soft16Params P) {
 #pragma unroll
           for (int v = 0; v < NS; ++v) acc[v] += g[v];
         };
-        if constexpr (CACHE || !EXACT) {
+        if constexpr (CACHE || !EXACT || (CODE == CODE_TABLE && V == 1)) {
 #pragma unroll
           for (int q = 0; q < UPT; ++q) unit(q);
         } else {

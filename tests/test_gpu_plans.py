@@ -174,3 +174,46 @@ def test_noalloc_holds_its_slots_in_two_halves(bcjr_mod, N, B):
         with_ws, without = ms(0), ms(1)
         _say(f"8 sequences: {with_ws:.3f} ms with a workspace, {without:.3f} ms without")
         assert without < 1.5 * with_ws
+
+
+@pytest.mark.parametrize("L", [15, 16])
+def test_low_temperature_tables_in_two_halves(bcjr_mod, oracle, L):
+    """A table at k = 2, V = 1 and T below the low-temperature line (0.08): the parity
+    bounds, and about the time of T = 0.1 (its codewords are held over the sweep
+    there too; read again for every unit, forward and entropy took twice as long)."""
+    from bcjr import ops
+    cb = _codebook(bcjr_mod, "table", L, 1)
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, 2, 1, torch.device("cuda"))
+    rng = np.random.default_rng(L)
+    B, N = 4, 16
+    x, g = (rng.standard_normal((B, N, 1)).astype(np.float32) for _ in range(2))
+    xd, gd = (torch.tensor(a, device="cuda") for a in (x, g))
+    for T in (0.06, 0.02):
+        _say(f"table L={L} T={T}")
+        soft, logZ = ops.forward(spec, xd, T, table)
+        H = ops.forward_entropy(spec, xd, T, table)[2]
+        d = ops.backward(spec, xd, T, table, gd)
+        cb_np = cb.cpu().numpy()
+        s_ref, z_ref = oracle.bcjr_forward(x, cb_np, T, L, 2)
+        assert max_rel(soft.cpu().numpy(), s_ref) < 1e-4 and max_rel(logZ.cpu().numpy(), z_ref) < 1e-5
+        assert max_rel(d.cpu().numpy(), oracle.bcjr_backward(x, cb_np, T, L, 2, g)) < 1e-3
+        h_ref = oracle.marginal_entropy(x, cb_np, T, L, 2)
+        assert np.abs(H.cpu().numpy() - h_ref).max() < 1e-4 * max(1.0, h_ref.max())
+
+    x = torch.randn(8, 96, 1, device="cuda", generator=torch.Generator("cuda").manual_seed(L))
+
+    def ms(f):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            f()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    for name, f in (("forward", ops.forward), ("entropy", ops.forward_entropy)):
+        warm, low = ms(lambda: f(spec, x, 0.1, table)), ms(lambda: f(spec, x, 0.06, table))
+        _say(f"{name} L={L}: {warm:.3f} ms at T = 0.1, {low:.3f} at T = 0.06")
+        assert low < 1.5 * warm
