@@ -477,22 +477,61 @@ size_t halves_bytes(const bcjr_problem* p, int op) {
          round256(((size_t)p->N + 2) * sizeof(double));
 }
 
+// Fewest steps that take two halves: below, the second launch costs more than the
+// steps it saves (one call among others, one launch -> two halves: 8 steps at L <= 12
+// 15-17 -> 18-20 us, their k V = 2 backward 21-24 -> 18-25; 16 steps 19-38 -> 18-39;
+// L = 14 and 16, 128 sequences, 4 steps 21-80 -> 25-85, 8 steps 33-135 -> 31-122; kV =
+// 4, L = 8, 4 steps 15-16 -> 18-19, 8 steps 21-25 -> 19-20; L >= 12, 2 steps 15-79 ->
+// 18-100, 4 steps 20-132 -> 19-127; L = 16, k = 1, V = 2, 4 steps 78-118 -> 53-89).
+long long halves_min_steps(const bcjr_problem* p, int op) {
+  const int KV = p->k * p->V;
+  if (KV == 4) return p->L >= 12 ? 4 : 8;
+  if (p->L == 16 && (p->V == 2 || op == OP_FWD_ENTROPY)) return 4;
+  return p->L >= 14 || (KV == 2 && op == OP_BWD) ? 8 : 16;
+}
+
+// Largest load of the kV <= 2 halves, in quarters of a workgroup per CU.  A lane per
+// output forms a butterfly's inputs once per output, so where one launch fills whole
+// waves (kV = 1 from L = 8, kV = 2 at L = 10) or a table of two components is read
+// that often, the halves lose their lead at 32 waves per CU (forward, N = 96, one
+// launch -> two halves: kV = 1, L = 11, 128 sequences 1.46 times as fast, 192 0.80;
+// L = 10, 768 sequences 1.18, 1,024 0.82; L = 9, whose waves one launch half fills,
+// 2,048 1.05).  Whole butterflies of two components, whose codewords no register
+// holds: up to 12 waves per CU, or the one workgroup of L >= 13 (HYB, L = 12, 384
+// sequences 1.16, 512 0.96; L = 13, 128 1.41, 192 0.93; a table at L = 13 1.11 and
+// 0.75), and a table's plain forward a little less (T = 0.06: L = 14, 96 sequences
+// 0.99, 128 0.91; L = 12, 128 1.16, 192 0.97; L = 16, 128 1.49).
+int halves_quarters_per_cu(const bcjr_problem* p, int op, const HalvesShape& sh) {
+  const int waves = sh.nthr / 64;
+  const bool table2 = p->V == 2 && p->code == BCJR_CODE_TABLE;
+  if (sh.lpb > 1) {
+    const bool early = p->k * p->V == 1 || p->L == 10 || (table2 && op != OP_BWD);
+    return 4 * ((waves > 1 && early ? 24 : 32) / waves);
+  }
+  if (p->V == 1) return 4 * (32 / waves);
+  if (table2 && op == OP_FWD) return p->L == 12 || p->L == 16 ? 4 : 3;
+  return 4 * std::max(1, 12 / waves);
+}
+
 // Whether a soft call runs its sequences in two halves each (bcjr_soft16.h,
 // bcjr_halves.h), and on which plan: when twice as many workgroups still all fit
 // at once, so that the steps in sequence are halved and no sequence waits for
-// another.  A sequence's last bits therefore depend on the batch it is in: the two
-// forms sum in other orders.  Every workspace of the queried size, and every
-// shorter one that takes several rounds, gives the same bits; one too short for
-// that (launch_halves) runs in one launch, with the bits of a large batch.  kV = 4: the plan of one launch, or, column walk, one workgroup of twice
-// the threads per CU where that is all there is.
+// another, and the two limits above say that it pays.  A sequence's last bits
+// therefore depend on the batch it is in: the two forms sum in other orders.  Every
+// workspace of the queried size, and every shorter one that takes several rounds,
+// gives the same bits; one too short for that (launch_halves) runs in one launch,
+// with the bits of a large batch.  kV = 4: the plan of one launch, or, column walk,
+// one workgroup of twice the threads per CU where that is all there is.
 // Measured, forward and backward, one launch -> two halves, N = 128: column walk
 // 8 sequences 1.17 -> 0.62 and 1.83 -> 0.85 ms (narrow workgroup 0.70 and 1.01),
 // 128 sequences 1.27 -> 0.70 and 1.95 -> 0.98 ms (0.79 and 1.11), 256 sequences on
 // the narrow one 1.28 -> 1.07 and 1.97 -> 1.61 ms; a table, 128 sequences 2.44 ->
 // 1.15 and 2.51 -> 1.43 ms; L = 12, 256 sequences 0.38 -> 0.26 and 0.42 -> 0.29 ms.
+// kV = 4 gains up to all that is resident (L = 8, 10, 12, 14: 2,048, 1,536, 512, 512
+// sequences 1.12, 1.39, 1.19, 1.17 times as fast).
 int halves_plan(const bcjr_problem* p, int op, const Plan& pl, Plan* out, bool* halves) {
   *halves = false;
-  if (p->N < 2) return BCJR_OK;
+  if (p->N < halves_min_steps(p, op)) return BCJR_OK;
   if (pl.KV == 4) {
     *halves = 2 * p->B <= pl.max_blocks;
     *out = pl;
@@ -500,8 +539,8 @@ int halves_plan(const bcjr_problem* p, int op, const Plan& pl, Plan* out, bool* 
       return make_plan(p, op, out, true);
     return BCJR_OK;
   }
-  // no plan is made for a batch that 32 waves a CU could not hold
-  if (2 * p->B > (long long)pl.num_cu * (2048 / halves_shape(p).nthr)) return BCJR_OK;
+  // (no plan is made for a batch beyond the limit; of pl only the CU count counts)
+  if (8 * p->B > (long long)pl.num_cu * halves_quarters_per_cu(p, op, halves_shape(p))) return BCJR_OK;
   const int rc = make_plan(p, op, out, true);
   if (rc || !out->fits) return rc;  // the LDS does not hold this N (or Q): one launch
   *halves = 2 * p->B <= out->max_blocks;
@@ -714,6 +753,12 @@ int bcjr_workspace_bytes(const bcjr_problem* prob, int op, size_t* bytes) {
     bool halves = false;
     rc = halves_plan(prob, op, pl, &hp, &halves);
     if (rc) return rc;
+    // The forward's workspace is the entropy's too, which takes larger batches in two
+    // halves at kV <= 2.
+    if (op == OP_FWD && !halves && pl.KV <= 2) {
+      rc = halves_plan(prob, OP_FWD_ENTROPY, pl, &hp, &halves);
+      if (rc) return rc;
+    }
     if (halves) *bytes = std::max(*bytes, (size_t)prob->B * halves_bytes(prob, op));
   }
   *bytes += table16_bytes(prob);

@@ -217,3 +217,51 @@ def test_low_temperature_tables_in_two_halves(bcjr_mod, oracle, L):
         warm, low = ms(lambda: f(spec, x, 0.1, table)), ms(lambda: f(spec, x, 0.06, table))
         _say(f"{name} L={L}: {warm:.3f} ms at T = 0.1, {low:.3f} at T = 0.06")
         assert low < 1.5 * warm
+
+
+# (k, V, L, code, op, N, sequences per 256 CUs up to which the batch runs in two halves; 0: never)
+@pytest.mark.parametrize("k,V,L,code,op,N,top", [
+    # a lane per output, 24 waves per CU where one launch fills its waves
+    (1, 1, 11, "table", 0, 64, 128), (1, 1, 11, "table", 1, 64, 128), (1, 1, 10, "table", 0, 64, 384),
+    (1, 1, 8, "table", 0, 64, 1536), (2, 1, 10, "1mad", 0, 64, 768), (2, 1, 10, "1mad", 1, 64, 768),
+    (2, 1, 11, "1mad", 0, 64, 512), (1, 2, 11, "table", 0, 64, 384),
+    # whole butterflies, codewords in registers or not
+    (1, 2, 12, "table", 0, 64, 384), (1, 2, 12, "table", 1, 64, 384),
+    (1, 2, 13, "table", 0, 64, 128), (1, 2, 13, "table", 1, 64, 128), (1, 2, 14, "table", 0, 64, 128),
+    (2, 1, 16, "3inst", 0, 64, 128),
+    # fewest steps
+    (2, 1, 10, "1mad", 0, 15, 0), (2, 1, 10, "1mad", 0, 16, 768), (2, 1, 10, "1mad", 1, 7, 0), (2, 1, 10, "1mad", 1, 8, 768),
+    (1, 1, 8, "table", 1, 15, 0), (2, 1, 16, "3inst", 1, 7, 0), (2, 1, 16, "3inst", 0, 8, 128), (4, 1, 14, "1mad", 0, 3, 0),
+    (4, 1, 16, "1mad", 1, 4, 128)])
+def test_where_two_halves_end(bcjr_mod, k, V, L, code, op, N, top):
+    """The largest batch that runs in two halves, from the workspace the call asks
+    for (the halves' state beside the slots; the forward's is also the entropy's,
+    whose lines lie at or above it): past these lines, or below these steps,
+    the halves were slower than one launch."""
+    from bcjr import _lib
+    lib = _lib.load()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    st, nt = op + 1, 1 << (L - k * V)
+    up = lambda b: (b + 255) // 256 * 256
+    halves = up(N * nt * 4 * st) + up(2 * st * nt * 4) + up(8 * (N + 2))
+    kind = {"table": _lib.CODE_TABLE, "1mad": _lib.CODE_1MAD, "3inst": _lib.CODE_3INST}[code]
+    top = top * cus // 256
+    for B, expect in ((max(top, 1), top > 0), (top + 1, False)):
+        rc, nbytes, _ = _query_seconds(lib, _lib.Problem(L, k, V, B, N, kind, 9, 0), op)
+        _say(f"k={k} V={V} L={L} {code} op {op} N={N} B={B}: {nbytes} bytes")
+        assert rc == 0 and (nbytes >= B * halves) == expect
+
+
+@pytest.mark.parametrize("L,top", [(12, 128), (14, 96)])
+def test_where_two_halves_end_for_a_table_of_two_components(bcjr_mod, L, top):
+    """The plain forward's own line there: a sequence has the bits of a batch far past
+    it from one sequence past it on, and not at it."""
+    from bcjr import ops
+    top = top * torch.cuda.get_device_properties(0).multi_processor_count // 256
+    cb = _codebook(bcjr_mod, "table", L, 2)
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, 1, 2, torch.device("cuda"))
+    x = torch.randn(8 * top, 32, 2, device="cuda", generator=torch.Generator("cuda").manual_seed(L))
+    _say(f"table V=2 L={L} forward around {top} sequences")
+    far, at, past = (ops.forward(spec, x[:B], 0.1, table)[0][:top] for B in (8 * top, top, top + 1))
+    assert torch.equal(far, past) and not torch.equal(far, at)
+    assert max_rel(at.cpu().numpy(), far.cpu().numpy()) < 1e-4  # the parity bound of soft

@@ -55,7 +55,8 @@ def _check(bcjr, oracle, kind, L, V, N, B, T, rows):
 
 @pytest.mark.parametrize("kind,V", [("hyb", 2), ("table", 2), ("table", 1), ("3inst", 1), ("1mad", 1)])
 @pytest.mark.parametrize("L,N,T", [(8, 1, 0.3), (9, 2, 0.06), (10, 3, 0.3), (11, 37, 0.1), (12, 16, 0.06), (13, 5, 0.2),
-                                   (14, 4, 0.06), (15, 9, 0.1), (16, 1, 0.2), (16, 2, 0.05), (16, 7, 0.1)])
+                                   (14, 4, 0.06), (15, 9, 0.1), (16, 1, 0.2), (16, 2, 0.05), (16, 7, 0.1),
+                                   (9, 6, 0.06), (10, 4, 0.3), (16, 4, 0.05)])
 def test_every_L_and_short_N(bcjr_mod, oracle, kind, V, L, N, T):
     print(f"[soft16] {kind} V={V} L={L} N={N} T={T}", flush=True)
     _check(bcjr_mod, oracle, kind, L, V, N, 3, T, [0, 1, 2])
@@ -130,7 +131,11 @@ def test_short_workspaces(bcjr_mod, oracle, kind, V):
                                           ("3inst", 2, 1, 12, 40), ("1mad", 2, 1, 13, 21), ("3inst", 2, 1, 14, 8),
                                           ("table", 2, 1, 15, 9), ("3inst", 2, 1, 16, 11), ("1mad", 2, 1, 16, 1),
                                           ("hyb", 1, 2, 8, 7), ("table", 1, 2, 12, 30), ("hyb", 1, 2, 13, 5),
-                                          ("table", 1, 2, 15, 4), ("hyb", 1, 2, 16, 6)])
+                                          ("table", 1, 2, 15, 4), ("hyb", 1, 2, 16, 6),
+                                          # (from the fewest steps that take two halves on)
+                                          ("table", 1, 1, 2, 18), ("table", 1, 1, 4, 16), ("3inst", 2, 1, 4, 17),
+                                          ("1mad", 2, 1, 6, 16), ("hyb", 1, 2, 8, 23), ("hyb", 1, 2, 13, 17),
+                                          ("table", 1, 2, 15, 12), ("table", 2, 1, 16, 8)])
 @pytest.mark.parametrize("T", [0.06, 0.2])
 def test_small_steps_in_two_halves(bcjr_mod, oracle, kind, k, V, L, N, T):
     """kV <= 2 (csrc/bcjr_halves.h): every L's launch shape, odd and even N, a
