@@ -29,6 +29,7 @@
 
 #include "bcjr_device.h"
 #include "bcjr_kernels.h"
+#include "bcjr_soft_common.h"
 
 namespace bcjr {
 
@@ -390,40 +391,6 @@ __global__ __launch_bounds__(1024, 4) void bcjr_halves_kernel(Soft16Params P) {
     return off;
   };
 
-  // log2 Z = C + D + LSE2(m~ + n~) where the sweeps meet and, GRAD, E[F] =
-  // sum_j P(j) (mu + nu)(j); the two vectors share one LDS layout.
-  auto meet = [&](const float* other, double CD) __attribute__((always_inline)) {
-    float mx = -INFINITY;
-    for (int j = tid; j < NT; j += nthr) mx = fmaxf(mx, stv[ST * j] + other[ST * j]);
-    mx = wave_max(mx);
-    if (lane == 0) wsum[wave] = mx;
-    __syncthreads();
-    float Mz = -INFINITY;
-    for (int w = 0; w < nwaves; ++w) Mz = fmaxf(Mz, wsum[w]);
-    float ps = 0.0f, pe = 0.0f;
-    for (int j = tid; j < NT; j += nthr) {
-      const float e = fexp2(stv[ST * j] + other[ST * j] - Mz);
-      ps += e;
-      if constexpr (GRAD) pe = fmaf(e, stv[2 * j + 1] + other[2 * j + 1], pe);
-    }
-    ps = wave_sum(ps);
-    if constexpr (GRAD) pe = wave_sum(pe);
-    __syncthreads();
-    if (lane == 0) {
-      wsum[wave] = ps;
-      wsum[kMaxWaves + wave] = pe;
-    }
-    __syncthreads();
-    float Ssum = 0.0f, Esum = 0.0f;
-    for (int w = 0; w < nwaves; ++w) {
-      Ssum += wsum[w];
-      if constexpr (GRAD) Esum += wsum[kMaxWaves + w];
-    }
-    logZ2 = CD + (double)Mz + (double)flog2(Ssum);
-    if constexpr (GRAD) EFg = Esum / Ssum - gZ;
-    __syncthreads();
-  };
-
   auto run = [&](auto exact) __attribute__((always_inline)) {
     using F = std::false_type;
     using Y = std::true_type;
@@ -452,7 +419,9 @@ __global__ __launch_bounds__(1024, 4) void bcjr_halves_kernel(Soft16Params P) {
     const int lo = role ? 0 : h, hi = role ? h : N;
     for (int i = lo + tid; i < hi; i += nthr) ovec[i] = moff[i];
     __syncthreads();
-    meet(mid + (size_t)(1 - role) * ST * NT, moff[N] + moff[N + 1]);
+    const SoftMeet z = soft_meet<GRAD>(stv, mid + (size_t)(1 - role) * ST * NT, NT, moff[N] + moff[N + 1], gZ, wsum);
+    logZ2 = z.logZ2;
+    EFg = z.EFg;
     if (role == 0) sweep(F{}, Y{}, exact, h, N - h, moff[N], 0.0f);
     else sweep(Y{}, Y{}, exact, h - 1, h, moff[N + 1], 0.0f);
     if (!GRAD && role == 0 && tid == 0 && P.logZ) P.logZ[b] = (float)(logZ2 * kLn2);

@@ -50,6 +50,7 @@
 
 #include "bcjr_device.h"
 #include "bcjr_kernels.h"
+#include "bcjr_soft_common.h"
 
 namespace bcjr {
 
@@ -450,9 +451,12 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
               hi = {far ? q.x : q.y, 0.0f, 0.0f, 0.0f};
             }
           };
-          auto path_value = [&](int i, const Cell& c) -> float {  // GRAD: z of input i
+          // GRAD: z of input i.  f = sg . h is formed first, as the storing sweep's table
+          // has it, and rounded once onto mu, which is the larger: two roundings at mu's
+          // size add 1.7 % to the gradient's error, the second operation 1.3 % to the time.
+          auto path_value = [&](int i, const Cell& c) -> float {
             if constexpr (!GRAD) return 0.0f;
-            else if constexpr (MARG && kCol) return fmaf(sg[V - 1], c.hy, fmaf(sg[0], c.hx, mu[i]));
+            else if constexpr (MARG && kCol) return mu[i] + fmaf(sg[V - 1], c.hy, sg[0] * c.hx);
             else return mu[i] + c.f;
           };
           // Output o(j)'s bases for even and odd inputs (alpha).
@@ -584,9 +588,9 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
                     hv(c0[q], h0);
                     hv(c1[q], h1);
                     if constexpr (GRAD && MARG) {
-                      const float zx = fmaf(sg[0], c0[q].hx, mu[i]);
-                      z0 = fmaf(sg[V - 1], c0[q].hy, zx);
-                      z1 = fmaf(sg[V - 1], c1[q].hy, zx);
+                      const float fx = sg[0] * c0[q].hx;
+                      z0 = mu[i] + fmaf(sg[V - 1], c0[q].hy, fx);
+                      z1 = mu[i] + fmaf(sg[V - 1], c1[q].hy, fx);
                     } else if constexpr (GRAD) {
                       z0 = mu[i] + c0[q].f;
                       z1 = mu[i] + c1[q].f;
@@ -707,39 +711,10 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
       return off;
     };
 
-    // log2 Z = C + D + LSE2(m~ + n~) where the sweeps meet (other = null: at the
-    // end, n~ = 0) and, GRAD, E[F] = sum_j P(j) (mu + nu)(j).  `own` and `other`
-    // hold the two vectors element by element in one LDS layout.
     auto meet = [&](const float* own, const float* other, double CD) __attribute__((always_inline)) {
-      float mx = -INFINITY;
-      for (int j = tid; j < NT; j += nthr) mx = fmaxf(mx, own[ST * j] + (other ? other[ST * j] : 0.0f));
-      mx = wave_max(mx);
-      if (lane == 0) wsum[wave] = mx;
-      __syncthreads();
-      float Mz = -INFINITY;
-      for (int w = 0; w < nwaves; ++w) Mz = fmaxf(Mz, wsum[w]);
-      float ps = 0.0f, pe = 0.0f;
-      for (int j = tid; j < NT; j += nthr) {
-        const float e = fexp2(own[ST * j] + (other ? other[ST * j] : 0.0f) - Mz);
-        ps += e;
-        if constexpr (GRAD) pe = fmaf(e, own[2 * j + 1] + (other ? other[2 * j + 1] : 0.0f), pe);
-      }
-      ps = wave_sum(ps);
-      if constexpr (GRAD) pe = wave_sum(pe);
-      __syncthreads();
-      if (lane == 0) {
-        wsum[wave] = ps;
-        wsum[kMaxWaves + wave] = pe;
-      }
-      __syncthreads();
-      float Ssum = 0.0f, Esum = 0.0f;
-      for (int w = 0; w < nwaves; ++w) {
-        Ssum += wsum[w];
-        if constexpr (GRAD) Esum += wsum[kMaxWaves + w];
-      }
-      logZ2 = CD + (double)Mz + (double)flog2(Ssum);
-      if constexpr (GRAD) EFg = Esum / Ssum - gZ;
-      __syncthreads();
+      const SoftMeet z = soft_meet<GRAD>(own, other, NT, CD, gZ, wsum);
+      logZ2 = z.logZ2;
+      EFg = z.EFg;
     };
     auto fill_state = [&](float value) __attribute__((always_inline)) {
       for (int j = tid; j < NT; j += nthr) {

@@ -215,3 +215,25 @@ def test_viterbi_table_with_and_without_its_copy(bcjr_mod, oracle, L, k, V, N):
         assert torch.isnan(mse[3]) and torch.isinf(mse[4])
         res.append(walk.cpu().numpy())
     assert np.array_equal(res[0], res[1]) and res[0].min() >= 0 and res[0].max() < 1 << L
+
+
+@pytest.mark.parametrize("kind,B,bound", [("hyb", 600, 1.85e-5), ("table", 300, 1.08e-5)])
+def test_gradient_keeps_its_precision_beside_a_large_expected_path_value(bcjr_mod, oracle, kind, B, bound):
+    """Weights about 2 and upstream gradients about 4: E[F] is about 128, which is
+    taken off path values as large, and a rounding of E[F] beyond its last one shows
+    in the whole gradient.  Relative error (2-norm) against the float64 oracle; the
+    bound lies halfway between float sums of E[F] (2.23e-5 hyb, 1.33e-5 table) and
+    sums in double (1.48e-5 and 0.82e-5)."""
+    from bcjr import ops
+    print(f"[soft16] {kind} B={B}, large E[F]", flush=True)
+    L, N, V, T = 16, 8, 2, 0.2
+    cb = _codebook(bcjr_mod, kind, L, V, 16)
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, 2, V, torch.device("cuda"))
+    rng = np.random.default_rng(3)
+    x = (2 + 0.2 * rng.standard_normal((B, N, V))).astype(np.float32)
+    g = (4 + 0.1 * rng.standard_normal((B, N, V))).astype(np.float32)
+    d = ops.backward(spec, torch.tensor(x, device="cuda"), T, table, torch.tensor(g, device="cuda"))
+    ref = oracle.bcjr_backward(x, cb.cpu().numpy(), T, L, 4, g)
+    err = float(np.linalg.norm(d.cpu().numpy() - ref) / np.linalg.norm(ref))
+    print(f"[soft16] {kind}: {err:.3e}", flush=True)
+    assert err < bound
