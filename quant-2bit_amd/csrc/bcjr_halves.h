@@ -93,31 +93,9 @@ __global__ __launch_bounds__(1024, 4) void bcjr_halves_kernel(Soft16Params P) {
   const float* seqb = P.seq + (size_t)b * N * V;
   float* outb = P.out + (size_t)b * N * V;
 
-  // T must be finite and > 0, the weights and upstream gradients finite;
-  // otherwise the sequence's outputs are NaN.
-  if (tid == 0) *bflag = 0;
-  __syncthreads();
-  int bad = !(Tb > 0.0f && Tb < INFINITY) || !__builtin_isfinite(gZ);
-  for (int i = tid; i < N * V; i += nthr) {
-    const float w = seqb[i];
-    wbuf[i] = w;
-    bad |= !__builtin_isfinite(w);
-    if constexpr (GRAD) {
-      const float gg = P.g_soft[(size_t)b * N * V + i];
-      gbuf[i] = gg;
-      bad |= !__builtin_isfinite(gg);
-    }
-  }
-  if (bad) *bflag = 1;
   for (int i = tid; i < 2 * kMaxWaves; i += nthr) wmax[i] = -INFINITY;  // waves that do not exist
-  __syncthreads();
-  if (*bflag) {  // uniform: every thread reads the flag after the barrier
-    if (role == 0 && P.mode == SOFT_SECOND) {
-      for (int i = tid; i < N * V; i += nthr) outb[i] = NAN;
-      if (tid == 0 && !GRAD && P.logZ) P.logZ[b] = NAN;
-      if constexpr (ENT)
-        for (int i = tid; i < N; i += nthr) P.H_out[(size_t)b * N + i] = NAN;
-    }
+  if (!soft_inputs<GRAD>(seqb, P.g_soft + (GRAD ? (size_t)b * N * V : 0), N * V, Tb, gZ, wbuf, gbuf, bflag)) {
+    if (role == 0 && P.mode == SOFT_SECOND) soft_fill_nan<GRAD, ENT>(P, b, outb, N * V);
     return;
   }
   __syncthreads();  // the flag's words serve as wsum below
@@ -127,25 +105,8 @@ __global__ __launch_bounds__(1024, 4) void bcjr_halves_kernel(Soft16Params P) {
 
   // Result of step t from the per-wave partials in buffer par (wave 0).
   auto step_out = [&](int t, int par) __attribute__((always_inline)) {
-    const float* sp = apart + par * nwaves * NS;
-    if constexpr (GRAD) {
-      const float a0 = sum_of_waves(sp, nwaves, NS);
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const float a1 = sum_of_waves(sp + 1 + v, nwaves, NS);
-        if (lane == 0) outb[t * V + v] = twoT * (a1 - wbuf[t * V + v] * a0);
-      }
-    } else {
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const float a = sum_of_waves(sp + v, nwaves, NS);
-        if (lane == 0) outb[t * V + v] = a;
-      }
-      if constexpr (ENT) {
-        const float h = sum_of_waves(sp + V, nwaves, NS);
-        if (lane == 0) P.H_out[(size_t)b * N + t] = -h * (float)kLn2;
-      }
-    }
+    soft_step_out<GRAD, ENT, V>(apart + par * nwaves * NS, nwaves, wbuf + t * V, twoT, outb + t * V,
+                                ENT ? P.H_out + (size_t)b * N + t : nullptr);
   };
 
   // One sweep over steps t0, t0 + dt, ... (n of them), dt = +1 (alpha) or -1

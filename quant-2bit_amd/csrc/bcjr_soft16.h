@@ -55,7 +55,7 @@
 namespace bcjr {
 
 // Threads of a workgroup and waves per SIMD the instance is built for.
-template <int CODE, int LPB, bool GRAD>
+template <int CODE, int LPB>
 struct Soft16Shape {
   static constexpr bool kCol = CODE == CODE_HYB_COL;
   static constexpr int threads = LPB == 2 || LPB == 16 ? 512 : 1024;
@@ -63,7 +63,7 @@ struct Soft16Shape {
 };
 
 template <bool GRAD, int CODE, int V, int LPB, bool ENT>
-__global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Shape<CODE, LPB, GRAD>::waves)) void bcjr_soft16_kernel(Soft16Params P) {
+__global__ __launch_bounds__((Soft16Shape<CODE, LPB>::threads), (Soft16Shape<CODE, LPB>::waves)) void bcjr_soft16_kernel(Soft16Params P) {
   constexpr int KV = 4, R = 16, RO = R / LPB, UW = 64 / LPB;
   constexpr bool kCol = CODE == CODE_HYB_COL;
   constexpr int ST = GRAD ? 2 : 1;      // floats of a state element
@@ -134,30 +134,8 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
     float* outb = P.out + (size_t)b * N * V;
     const int role = P.mode == SOFT_WHOLE ? 0 : (int)(blockIdx.x & 1);  // two halves: 0 alpha, 1 beta
 
-    // T must be finite and > 0, the weights and upstream gradients finite;
-    // otherwise the sequence's outputs are NaN.
-    if (tid == 0) *bflag = 0;
-    __syncthreads();
-    int bad = !(Tb > 0.0f && Tb < INFINITY) || !__builtin_isfinite(gZ);
-    for (int i = tid; i < N * V; i += nthr) {
-      const float w = seqb[i];
-      wbuf[i] = w;
-      bad |= !__builtin_isfinite(w);
-      if constexpr (GRAD) {
-        const float gg = P.g_soft[(size_t)b * N * V + i];
-        gbuf[i] = gg;
-        bad |= !__builtin_isfinite(gg);
-      }
-    }
-    if (bad) *bflag = 1;
-    __syncthreads();
-    if (*bflag) {  // uniform: every thread reads the flag after the barrier
-      if (role == 0 && P.mode != SOFT_FIRST) {
-        for (int i = tid; i < N * V; i += nthr) outb[i] = NAN;
-        if (tid == 0 && !GRAD && P.logZ) P.logZ[b] = NAN;
-        if constexpr (ENT)
-          for (int i = tid; i < N; i += nthr) P.H_out[(size_t)b * N + i] = NAN;
-      }
+    if (!soft_inputs<GRAD>(seqb, P.g_soft + (GRAD ? (size_t)b * N * V : 0), N * V, Tb, gZ, wbuf, gbuf, bflag)) {
+      if (role == 0 && P.mode != SOFT_FIRST) soft_fill_nan<GRAD, ENT>(P, b, outb, N * V);
       __syncthreads();
       continue;
     }
@@ -168,25 +146,8 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
 
     // Result of step t from the per-wave partials in buffer par (wave 0).
     auto step_out = [&](int t, int par) __attribute__((always_inline)) {
-      const float* sp = apart + par * nwaves * NS;
-      if constexpr (GRAD) {
-        const float a0 = sum_of_waves(sp, nwaves, NS);
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-          const float a1 = sum_of_waves(sp + 1 + v, nwaves, NS);
-          if (lane == 0) outb[t * V + v] = twoT * (a1 - wbuf[t * V + v] * a0);
-        }
-      } else {
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-          const float a = sum_of_waves(sp + v, nwaves, NS);
-          if (lane == 0) outb[t * V + v] = a;
-        }
-        if constexpr (ENT) {
-          const float h = sum_of_waves(sp + V, nwaves, NS);
-          if (lane == 0) P.H_out[(size_t)b * N + t] = -h * (float)kLn2;
-        }
-      }
+      soft_step_out<GRAD, ENT, V>(apart + par * nwaves * NS, nwaves, wbuf + t * V, twoT, outb + t * V,
+                                  ENT ? P.H_out + (size_t)b * N + t : nullptr);
     };
 
     // One sweep over steps t0, t0 + dt, ... (n of them), dt = +1 (alpha) or -1
@@ -306,8 +267,7 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
         }
         const uint32_t tab = !GRAD && !MARG ? 12288u * (uint32_t)(t & 1) : 0u;
 
-        // State elements: element k = 0..15 of the butterfly at yb ^ Kk(k).
-        const uint32_t yb = state0 + 0u;
+        // State elements: element k = 0..15 of the butterfly at state0 + (yu ^ koff(k)).
         const uint32_t yu = el_off((uint32_t)ul, rho);
         uint32_t K1 = el_off((uint32_t)NB, rho), K2 = el_off((uint32_t)NB << 1, rho),
                  K4 = el_off((uint32_t)NB << 2, rho), K8 = el_off((uint32_t)NB << 3, rho);
@@ -319,11 +279,11 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
 #pragma unroll
         for (int q = 0; q < R; ++q) {
           if constexpr (GRAD) {
-            const float2 v2 = *reinterpret_cast<const float2*>(smem + yb + (yu ^ koff(q)));
+            const float2 v2 = *reinterpret_cast<const float2*>(smem + state0 + (yu ^ koff(q)));
             m[q] = v2.x;
             mu[q] = v2.y;
           } else {
-            m[q] = *reinterpret_cast<const float*>(smem + yb + (yu ^ koff(q)));
+            m[q] = *reinterpret_cast<const float*>(smem + state0 + (yu ^ koff(q)));
           }
         }
         // Codeword of output o(j), input i.  The lane's base and the strides are
@@ -358,11 +318,11 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
 #pragma unroll
             for (int j = 0; j < RO; ++j) {
               if constexpr (GRAD) {
-                const float2 v2 = *reinterpret_cast<const float2*>(smem + yb + (yo ^ koff(o_uni(j))));
+                const float2 v2 = *reinterpret_cast<const float2*>(smem + state0 + (yo ^ koff(o_uni(j))));
                 own[2 * j] = v2.x;
                 own[2 * j + 1] = v2.y;
               } else {
-                own[j] = *reinterpret_cast<const float*>(smem + yb + (yo ^ koff(o_uni(j))));
+                own[j] = *reinterpret_cast<const float*>(smem + state0 + (yo ^ koff(o_uni(j))));
               }
             }
             float* dst = slot + ((size_t)t * NB + ul) * (R * ST) + (size_t)o_lane * ST;
@@ -421,9 +381,9 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
           };
           auto put = [&](int j, float no, float nuo) __attribute__((always_inline)) {
             if constexpr (GRAD) {
-              *reinterpret_cast<float2*>(smem + yb + (yo ^ koff(o_uni(j)))) = make_float2(no, nuo);
+              *reinterpret_cast<float2*>(smem + state0 + (yo ^ koff(o_uni(j)))) = make_float2(no, nuo);
             } else {
-              *reinterpret_cast<float*>(smem + yb + (yo ^ koff(o_uni(j)))) = no;
+              *reinterpret_cast<float*>(smem + state0 + (yo ^ koff(o_uni(j)))) = no;
             }
             tmax = vmax_raw(tmax, no);
           };
@@ -771,5 +731,11 @@ __global__ __launch_bounds__((Soft16Shape<CODE, LPB, GRAD>::threads), (Soft16Sha
     __syncthreads();
   }
 }
+
+// The instances of one code, V and lanes per butterfly, by kind (bcjr_kernels.h).
+#define BCJR_SOFT16_KINDS(CODE_, V_, LPB_)                                                                    \
+  if (kind == 0) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, false>);    \
+  if (kind == 1) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<true, CODE_, V_, LPB_, false>);     \
+  return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, true>);
 
 }  // namespace bcjr

@@ -3,11 +3,6 @@
 
 namespace bcjr {
 
-#define BCJR_SOFT16_KINDS(CODE_, V_, LPB_)                                                                    \
-  if (kind == 0) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, false>);    \
-  if (kind == 1) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<true, CODE_, V_, LPB_, false>);     \
-  return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, true>);
-
 const void* soft16_col_kernel_ptr(int kind, int lpb) {
   if (lpb == 2) {
     BCJR_SOFT16_KINDS(CODE_HYB_COL, 2, 2)

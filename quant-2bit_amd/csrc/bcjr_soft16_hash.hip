@@ -3,11 +3,6 @@
 
 namespace bcjr {
 
-#define BCJR_SOFT16_KINDS(CODE_, V_, LPB_)                                                                    \
-  if (kind == 0) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, false>);    \
-  if (kind == 1) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<true, CODE_, V_, LPB_, false>);     \
-  return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, true>);
-
 const void* soft16_hash_kernel_ptr(int kind, int code, int lpb) {
   if (code == CODE_1MAD && lpb == 4) {
     BCJR_SOFT16_KINDS(CODE_1MAD, 1, 4)

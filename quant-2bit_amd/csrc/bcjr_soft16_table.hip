@@ -3,11 +3,6 @@
 
 namespace bcjr {
 
-#define BCJR_SOFT16_KINDS(CODE_, V_, LPB_)                                                                    \
-  if (kind == 0) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, false>);    \
-  if (kind == 1) return reinterpret_cast<const void*>(&bcjr_soft16_kernel<true, CODE_, V_, LPB_, false>);     \
-  return reinterpret_cast<const void*>(&bcjr_soft16_kernel<false, CODE_, V_, LPB_, true>);
-
 namespace {
 
 // out[(p * 16 + c) * NB + u] = table[p * NT + 16 u + c] (V floats each): states of

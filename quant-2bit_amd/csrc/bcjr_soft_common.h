@@ -8,6 +8,68 @@
 
 namespace bcjr {
 
+// Reads a sequence's inputs into LDS and checks them: T must be finite and > 0, the
+// weights and upstream gradients finite.  bflag is the workgroup's flag word; when it
+// is set the sequence's outputs are NaN (soft_fill_nan).  Uniform result.
+template <bool GRAD>
+__device__ __forceinline__ bool soft_inputs(const float* seq, const float* g_soft, int n, float T, float gZ, float* wbuf,
+                                            float* gbuf, int* bflag) {
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  if (tid == 0) *bflag = 0;
+  __syncthreads();
+  int bad = !(T > 0.0f && T < INFINITY) || !__builtin_isfinite(gZ);
+  for (int i = tid; i < n; i += nthr) {
+    const float w = seq[i];
+    wbuf[i] = w;
+    bad |= !__builtin_isfinite(w);
+    if constexpr (GRAD) {
+      const float gg = g_soft[i];
+      gbuf[i] = gg;
+      bad |= !__builtin_isfinite(gg);
+    }
+  }
+  if (bad) *bflag = 1;
+  __syncthreads();
+  return *bflag == 0;  // every thread reads the flag after the barrier
+}
+
+// The outputs of sequence b whose inputs are not finite.
+template <bool GRAD, bool ENT>
+__device__ __forceinline__ void soft_fill_nan(const Soft16Params& P, long long b, float* out, int n) {
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  for (int i = tid; i < n; i += nthr) out[i] = NAN;
+  if (tid == 0 && !GRAD && P.logZ) P.logZ[b] = NAN;
+  if constexpr (ENT)
+    for (int i = tid; i < P.N; i += nthr) P.H_out[(size_t)b * P.N + i] = NAN;
+}
+
+// Outputs of one step from its per-wave partials sp (wave 0): GRAD d seq of the step
+// (w its weights), else the soft codeword and, ENT, the entropy into *H.
+template <bool GRAD, bool ENT, int V>
+__device__ __forceinline__ void soft_step_out(const float* sp, int nwaves, const float* w, float twoT, float* out,
+                                              float* H) {
+  constexpr int NS = V + (GRAD || ENT ? 1 : 0);
+  const int lane = threadIdx.x & 63;
+  if constexpr (GRAD) {
+    const float a0 = sum_of_waves(sp, nwaves, NS);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const float a1 = sum_of_waves(sp + 1 + v, nwaves, NS);
+      if (lane == 0) out[v] = twoT * (a1 - w[v] * a0);
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const float a = sum_of_waves(sp + v, nwaves, NS);
+      if (lane == 0) out[v] = a;
+    }
+    if constexpr (ENT) {
+      const float h = sum_of_waves(sp + V, nwaves, NS);
+      if (lane == 0) *H = -h * (float)kLn2;
+    }
+  }
+}
+
 struct SoftMeet {
   double logZ2;  // log2 Z
   float EFg;     // E[F] - g_Z (GRAD)
