@@ -118,7 +118,9 @@ int bcjr_forward(const bcjr_problem* prob, const float* seq, const float* T,
  * (src/bcjr/forward_backward.py:230-231): marginals P (B, N, 2^L), log_alpha and
  * log_beta (B, N, 2^L), natural log, as the reference defines them
  * (log_alpha_{-1} = 0, log_beta_{N-1} = 0).  Meant for small B (the reference
- * uses it on <= 32 tiles, src/bcjr/anneal.py:143-184). */
+ * uses it on <= 32 tiles, src/bcjr/anneal.py:143-184).  soft and logZ are
+ * bcjr_forward's, up to the last bits for V = 1, kV = 2 from L = 14 on where the batch
+ * is too large for two halves. */
 int bcjr_forward_internals(const bcjr_problem* prob, const float* seq, const float* T,
                            const float* codebook_or_lut, float* soft, float* logZ,
                            float* marginals, float* log_alpha, float* log_beta,

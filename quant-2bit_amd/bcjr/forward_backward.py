@@ -193,6 +193,10 @@ def bcjr_forward_backward(sequences, codebook, T_temp,
     Returns (soft (B,N,V), log_Z (B,)), or with return_internals
     (soft, log_Z, P, log_alpha, log_beta) with the last three (B, N, 2^L).
     soft and log_Z are differentiable with respect to sequences in both forms.
+
+    A batch too small to fill the chip runs each sequence in two halves, whose
+    float32 sums take another order, so a sequence's last bits can differ with the
+    batch it is in; equal calls give equal bits.
     """
     _check_args(sequences, codebook, L, k, V, preds, succs)
     dt = sequences.dtype

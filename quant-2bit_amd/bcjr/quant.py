@@ -64,9 +64,11 @@ def bcjr_quantize_tiles(sequences, codebook, T_temp, preds=None, succs=None,
     Here one launch per direction covers the whole batch with memory bounded by
     the engine's workspace, and the node keeps only its inputs for the backward,
     so chunk_size and use_checkpoint are accepted for signature compatibility
-    and not applied: the result is the same (sequences are independent) and a
-    chunked loop would only multiply launches (a 237,568-tile layer at
-    chunk_size=8 would be ~30,000 of them, each filling 8 of 256 CUs)."""
+    and not applied: sequences are independent, so a chunked loop gives the same
+    result (up to the order of float32 sums: batches too small to fill the chip
+    run each sequence in two halves) and would only multiply launches (a
+    237,568-tile layer at chunk_size=8 would be ~30,000 of them, each filling 8
+    of 256 CUs)."""
     soft, _ = bcjr_forward_backward(sequences, codebook, T_temp, L=L, k=k, V=V,
                                     preds=preds, succs=succs)
     return soft

@@ -192,16 +192,18 @@ int make_plan(const bcjr_problem* p, int op, Plan* pl, bool wide = false) {
   return BCJR_OK;
 }
 
-// LDS bank conflicts of the backward kernel's in-place layout: element
-// S(rotr(k*NB + u, rho)) holds slot k of butterfly u, one 8-byte (m~, mu) pair,
-// read and written by the same lane.  Measured on gfx950: a 64-bit LDS read
+// LDS bank conflicts of an in-place layout: element S(rotr(k*NB + u, rho)) holds
+// slot k of butterfly u.  Priced for 8-byte (m~, mu) pairs read and written by one
+// lane per butterfly, the backward of kV <= 2.  Measured on gfx950: a 64-bit LDS read
 // serves each 32-lane half of a wave from 32 eight-byte banks (conflict-free
 // when the half's elements differ mod 32); a 64-bit write serves 16 lanes at a
 // time from 32 four-byte banks (conflict-free when each quarter's elements
 // differ mod 16).  One wave of butterflies (u = 0..63) suffices: higher bits of
-// u XOR the same constant into every element of the wave.  Returns the extra
-// passes summed over the rotations a sweep reaches (multiples of gcd(kV, nb))
-// and the slots.
+// u XOR the same constant into every element of the wave.  The kV = 4 kernels take
+// the same layouts: their lanes that share a butterfly read the same words, so a wave
+// touches 4 or 16 butterflies of those 64; the forward's floats are not priced.
+// Returns the extra passes summed over the rotations a sweep reaches (multiples of
+// gcd(kV, nb)) and the slots.
 int swizzle_cost(int L, int KV, const bcjr::Swizzle& s) {
   const int nb = L - KV, NB = 1 << (nb - KV), R = 1 << KV;
   const int lanes = std::min(NB, 64);
@@ -287,11 +289,12 @@ bcjr::Swizzle swizzle_of(int L, int KV) {
   return memo[L][KV];
 }
 
-// State layout of the column-walk backward instance (L = 16, kV = 4), whose
-// thread tid holds butterfly col_walk_unit(tid) rather than tid: with this
-// swizzle every half-wave's 64-bit reads and every quarter-wave's 64-bit writes
-// of S(rotr(k*NB + u, rho)) fall in distinct banks over all 256 lanes, the 16
-// slots and the rotations 0, 4, 8 (the search above assumes u = tid).
+// State layout of the column walk's (m~, mu) pairs (L = 16, kV = 4), whose lane
+// slot q holds butterfly col_walk_unit(q) rather than q: with this swizzle the 64-bit
+// reads of 32 consecutive slots and the 64-bit writes of 16 of S(rotr(k*NB + u, rho))
+// fall in distinct banks for all 256 slots, the 16 elements and the rotations 0, 4, 8
+// (the search above assumes u = q).  The column walk's forward lays its floats out
+// by col_walk_state_el.
 constexpr bcjr::Swizzle kColWalkSwizzle = {{4, 6, 8, 31}, {3u, 31u, 15u, 0u}};
 
 // Opts the plan's kernel in to its LDS and finds how many blocks the device holds.
@@ -843,8 +846,10 @@ int bcjr_forward_internals(const bcjr_problem* prob, const float* seq, const flo
   P.t_per_seq = prob->t_per_seq ? 1 : 0;
   rc = launch(pl, prob->B, ws_bytes, &P, stream);
   if (rc) return rc;
-  // soft and log Z as bcjr_forward gives them, bit for bit, where it runs other
-  // kernels than the diagnostics one (whose own values these overwrite).
+  // kV = 4 and batches in two halves: soft and log Z as bcjr_forward gives them, bit
+  // for bit, over the diagnostics kernel's own, which sums in another order (a forward
+  // more, 2-9 % of the call at L = 16, 20-40 % on the smallest lattices).  Larger
+  // kV <= 2 batches keep its own: the bits of bcjr_forward below L = 14 only.
   bcjr::Soft16Params S = {};
   S.seq = seq;
   S.T = T;

@@ -138,8 +138,11 @@ __device__ __forceinline__ float2 hyb_col_read(const unsigned char* lutb, uint32
 // state 16u + c is bits [6, 12) of x = s^2 + s for Q = 9 (the reference's LUT).
 // Over each coset of span(bits 2..7 of u) those columns are all 64 distinct, for
 // every c, so 64 slots own one coset: u takes q's bits 0..5 as its bits 2..7 and
-// q >> 6 as its bits 0, 1.  Then 32 slots' table reads hit distinct banks
-// (checked in tests/test_capi_cpu.py).  (A smaller Q has fewer columns.)
+// q >> 6 as its bits 0, 1.  Then the table reads of 16 consecutive slots (16-byte
+// entries) and of 32 (8 bytes) hit distinct banks (checked in
+// tests/test_capi_cpu.py); at four lanes per butterfly half a wave reads 8-byte
+// entries of two outputs, 16 slots each, and two of them can share a bank.  (A
+// smaller Q has fewer columns.)
 __host__ __device__ constexpr uint32_t col_walk_unit(uint32_t tid) {
   return ((tid >> 6) & 3u) | ((tid & 63u) << 2);
 }

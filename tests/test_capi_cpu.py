@@ -275,15 +275,15 @@ def _distinct_in_groups(el, group, banks):
 
 
 def test_column_walk_layouts_are_bank_conflict_free():
-    """Column-walk soft kernels (L=16, kV=4, 256 threads, thread tid on butterfly
-    u = col_walk_unit(tid)), under gfx950's LDS banking: 64-bit reads serve each
-    half-wave from 32 eight-byte banks, 64-bit writes each quarter-wave from 32
-    four-byte banks, 32-bit reads 64 lanes from 64 banks, 32-bit writes 32 lanes
-    from 32 banks.  Checked: the LUT gathers at Q = 9 (bank = bits [6, 11) of
-    r^2 + r, r = 16u + c), the 32-bit reads of the per-step emission tables in
-    the LUT's layout (bank = bits [6, 12)), and the in-place state vectors at the
-    rotations 0, 4, 8: the forward's floats (col_walk_state_el, 32-bit) and the
-    backward's swizzled (m~, mu) pairs (64-bit)."""
+    """Column-walk kernels (L=16, kV=4; lane slot q on butterfly u = col_walk_unit(q)),
+    under gfx950's LDS banking: 64-bit reads serve 32 lanes from 32 eight-byte banks,
+    64-bit writes 16 lanes from 32 four-byte banks, 32-bit reads 64 lanes from 64
+    banks, 32-bit writes 32 lanes from 32 banks.  Checked for consecutive slots: the
+    8-byte reads of a LUT or per-step table at Q = 9 (bank = bits [6, 11) of r^2 + r,
+    r = 16u + c), its 4-byte reads (bank = bits [6, 12)), and the in-place state
+    vectors at the rotations 0, 4, 8: the forward's floats (col_walk_state_el, 32-bit)
+    and the backward's swizzled (m~, mu) pairs (64-bit).  (The 16-byte entries:
+    test_column_walk_pair_entries.)"""
     M = _col_walk_maps()
     tid = np.arange(256, dtype=np.int64)
     U = M["col_walk_unit"](tid)
@@ -312,6 +312,58 @@ def test_column_walk_layouts_are_bank_conflict_free():
             assert np.array_equal(E(x), E(rotr(U, rho)) ^ E(rotr(np.full_like(U, 256 * k), rho)))
             assert _distinct_in_groups(E(x), 64, 64) and _distinct_in_groups(E(x), 32, 32), (rho, k)
             assert _distinct_in_groups(S(x), 32, 32) and _distinct_in_groups(S(x), 16, 16), (rho, k)
+
+
+@pytest.mark.parametrize("lpb", [2, 4])
+def test_column_walk_pair_entries(lpb):
+    """The column-walk soft kernels' per-step tables (24 rows of 64 entries of 16 bytes,
+    rows 8..15 of rows 0..7's LUT entries with the sign of the second component
+    flipped, rows 16..23 as 0..7): a lane's base plus hyb_pair_step(p, c), p < 8, stays
+    below row 24 and is the entry of state p * 4096 + 16u + c and, 8 rows on, of that
+    with p + 8, or with hyb_pair_far the other way round; in both directions, for every
+    lane and lanes per butterfly.  A pass of 16 lanes reads 16 entries (16 bytes) of
+    distinct banks, and at two lanes per butterfly one of 32 lanes 32 entries of 8."""
+    Q, RO, H = 9, 16 // lpb, 8 // lpb
+    slot = np.arange(256, dtype=np.int64)
+    U = _col_walk_maps()["col_walk_unit"](slot)
+    col_base = lambda r: ((((r * r + r) >> (15 - Q)) & ((1 << (Q - 3)) - 1)) << 3) | ((((r * r + r) >> 12) & 15) << 9)
+    step = lambda p, c: ((p * (2 * c + 1)) & 7) << 10
+    far = lambda p, c: (p * (2 * c + 1)) & 8
+
+    def signed_index(p, r):
+        s = p * 4096 + r
+        return ((s * s + s) >> (15 - Q)) & ((2 << Q) - 1)
+
+    def check(byte, p, c, r):  # r = 16u + c of the lane's state, byte its entry for p and p + 8
+        assert (byte & 15).max() == 0 and (byte >> 10).max() < 24
+        row, column = byte >> 10, (byte >> 4) & 63
+        for pp, rows_on in ((p, 0), (p + 8, 8)):
+            want = signed_index(pp, r)
+            assert np.array_equal(column, want & 63)
+            assert np.array_equal((row + rows_on + far(p, c)) & 15, want >> 6)
+        assert _distinct_in_groups(byte >> 4, 16, 16)
+        if lpb == 2:
+            assert _distinct_in_groups(byte >> 4, 32, 32)
+
+    for part in range(lpb):
+        for i in range(8):  # alpha: inputs p = i and i + 8 of output j + RO * part
+            for j in range(RO):
+                c = j + RO * part
+                e = col_base(16 * U + c) << 1
+                rows = 8 * (part & 1) if lpb == 4 and i & 1 else 0
+                base = (e & 1023) | ((e + (rows << 10)) & 0x3C00)
+                check(base + step(i, j), i, j, 16 * U + c)
+        for j in range(H):  # beta: outputs j + H * part and 8 on, of input c
+            for c in range(16):
+                e = col_base(16 * U + c) << 1
+                base = (e & 1023) | ((e + ((H * part * (2 * c + 1)) << 10)) & 0x3C00)
+                byte, p = base + step(j, c), j + H * part
+                row, column = byte >> 10, (byte >> 4) & 63
+                assert row.max() < 24 and _distinct_in_groups(byte >> 4, 16, 16)
+                for pp, rows_on in ((p, 0), (p + 8, 8)):
+                    want = signed_index(pp, 16 * U + c)
+                    assert np.array_equal(column, want & 63)
+                    assert np.array_equal((row + rows_on + far(j, c)) & 15, want >> 6)
 
 
 # ------------------------- contract checks (no device) -------------------------

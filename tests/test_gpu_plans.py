@@ -265,3 +265,23 @@ def test_where_two_halves_end_for_a_table_of_two_components(bcjr_mod, L, top):
     far, at, past = (ops.forward(spec, x[:B], 0.1, table)[0][:top] for B in (8 * top, top, top + 1))
     assert torch.equal(far, past) and not torch.equal(far, at)
     assert max_rel(at.cpu().numpy(), far.cpu().numpy()) < 1e-4  # the parity bound of soft
+
+
+@pytest.mark.parametrize("kind,k,V,L,B,same", [("hyb", 2, 2, 16, 2, True), ("table", 4, 1, 9, 700, True), ("1mad", 2, 1, 14, 4, True),
+                                               ("1mad", 2, 1, 12, 1200, True), ("1mad", 2, 1, 14, 160, False)])
+def test_diagnostics_give_the_forwards_soft_and_log_z(bcjr_mod, kind, k, V, L, B, same):
+    """return_internals: soft and log Z are the plain forward's bit for bit, in two
+    halves, at kV = 4 and in one launch below L = 14; from there on (kV = 2, V = 1) the
+    plain forward of a large batch runs on twice the threads, and they agree to the
+    parity bounds."""
+    from bcjr import ops
+    cb = _codebook(bcjr_mod, kind, L, V)
+    spec, table = bcjr_mod.codes.resolve_codebook(cb, L, k, V, torch.device("cuda"))
+    x = torch.randn(B, 16, V, device="cuda", generator=torch.Generator("cuda").manual_seed(B))
+    _say(f"diagnostics {kind} L={L} kV={k * V} B={B}")
+    soft, logZ = ops.forward(spec, x, 0.2, table)
+    got = ops.forward_internals(spec, x, 0.2, table)
+    if same:
+        assert torch.equal(got[0], soft) and torch.equal(got[1], logZ)
+    assert max_rel(got[0].cpu().numpy(), soft.cpu().numpy()) < 1e-4
+    assert max_rel(got[1].cpu().numpy(), logZ.cpu().numpy()) < 1e-5
