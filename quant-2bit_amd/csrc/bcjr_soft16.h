@@ -38,13 +38,13 @@
 // 5.06 against 17.3 ms).  The other codes hash each state, HYB through the LUT in
 // LDS.
 //
-// Bounds.  Large batches: VALU issue (column walk, L = 16, T = 0.1: 9.6 VALU
-// instructions per cell forward and 17.2 backward in the step bodies, plus about
-// 190 per wave and step), then the tables' barrier; small ones: the latency of a
-// step, N/2 of them each way.  Measured against one 256-thread workgroup per
+// Bounds.  Large batches: VALU issue (column walk, L = 16, T = 0.1: 11.8 VALU
+// instructions per cell forward, 2.3 of them transcendental, and 20.5 backward),
+// LDS latency and the tables' barrier; small ones: the latency of a step, N/2 of
+// them each way.  Measured against one 256-thread workgroup per
 // sequence with a butterfly per lane, at N = 128, HYB Q = 9: 8 sequences forward
-// 1.61 -> 0.62 ms, backward 2.67 -> 0.85 ms; 4,096 sequences 15.4 -> 13.5-14.3 ms
-// and 24.5 -> 23.6 ms; L = 12, 128 sequences (16 butterflies) 2.71 -> 0.21 ms and
+// 1.61 -> 0.62 ms, backward 2.67 -> 0.85 ms; 4,096 sequences 15.4 -> 14.1-14.3 ms
+// and 24.5 -> 24.0-24.6 ms; L = 12, 128 sequences (16 butterflies) 2.71 -> 0.21 ms and
 // 3.62 -> 0.24 ms; a table at L = 16, 500 sequences 24.7 -> 4.9 and 24.0 -> 5.1 ms.
 #pragma once
 
